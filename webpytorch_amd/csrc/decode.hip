@@ -430,57 +430,6 @@ __global__ __launch_bounds__(256) void attention_decode_small_kernel(
   if (tid < HD) out[(size_t)h * HD + tid] = ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
 }
 
-// Causal grouped-query attention: token t (position pos0 + t) of query head h attends to
-// cache positions 0 .. pos0 + t of kv head h / (NH / NKV). One wave per (head, token):
-// lanes over positions for the scores, lanes over the head dimension for the output.
-// scores = (q . k) * scale; p = exp(s - max) / sum; out = sum p v.
-__global__ __launch_bounds__(64) void attention_kernel(const float* __restrict__ q, const float* __restrict__ kc,
-                                                       const float* __restrict__ vc, const int32_t* __restrict__ state,
-                                                       float* __restrict__ out, int NH, int NKV, int HD, int LMAX,
-                                                       float scale) {
-  extern __shared__ float sp[];  // [LMAX] scores, then probabilities
-  __shared__ float qs[256];
-  const int h = blockIdx.x, t = blockIdx.y;
-  const int lane = threadIdx.x;
-  const int kv = h / (NH / NKV);
-  int S = state[0] + t + 1;
-  S = S > LMAX ? LMAX : S;
-  for (int d = lane; d < HD; d += 64) qs[d] = q[((size_t)t * NH + h) * HD + d];
-  __syncthreads();
-  const float* K = kc + (size_t)kv * LMAX * HD;
-  const float* Vv = vc + (size_t)kv * LMAX * HD;
-  float mx = -INFINITY;
-  for (int j = lane; j < S; j += 64) {
-    const float* kr = K + (size_t)j * HD;
-    float a = 0.f;
-    for (int d = 0; d < HD; d += 4) {
-      const float4 k4 = *reinterpret_cast<const float4*>(kr + d);
-      a = fmaf(qs[d], k4.x, a);
-      a = fmaf(qs[d + 1], k4.y, a);
-      a = fmaf(qs[d + 2], k4.z, a);
-      a = fmaf(qs[d + 3], k4.w, a);
-    }
-    a *= scale;
-    sp[j] = a;
-    mx = fmaxf(mx, a);
-  }
-  mx = wave_max(mx);
-  float sum = 0.f;
-  for (int j = lane; j < S; j += 64) {
-    const float e = expf(sp[j] - mx);
-    sp[j] = e;
-    sum += e;
-  }
-  sum = wave_sum(sum);
-  for (int j = lane; j < S; j += 64) sp[j] = sp[j] / sum;
-  __syncthreads();
-  for (int d = lane; d < HD; d += 64) {
-    float o = 0.f;
-    for (int j = 0; j < S; ++j) o = fmaf(sp[j], Vv[(size_t)j * HD + d], o);
-    out[((size_t)t * NH + h) * HD + d] = o;
-  }
-}
-
 // out[t][i] = silu(gu[t][i]) * gu[t][I + i], silu(x) = x * (1 / (1 + exp(-x)))
 __global__ __launch_bounds__(256) void silu_mul_kernel(const float* __restrict__ gu, float* __restrict__ out, int I) {
   const int t = blockIdx.y;
@@ -644,19 +593,6 @@ extern "C" int miq_attention_decode(const float* qkv, const int32_t* state, cons
     hipLaunchKernelGGL(attention_decode_kernel, dim3(NH), dim3(256), (size_t)LMAX * 4, static_cast<hipStream_t>(stream),
                        qkv, state, cos_tab, sin_tab, kcache, vcache, out, NH, NKV, HD, LMAX, scale);
   return check_launch("attention_decode");
-}
-
-extern "C" int miq_attention(const float* q, const float* kcache, const float* vcache, const int32_t* state, float* out,
-                             int T, int NH, int NKV, int HD, int LMAX, float scale, void* stream) {
-  MIQ_REQUIRE(T >= 0 && NH > 0 && NKV > 0 && NH % NKV == 0 && HD > 0 && HD <= 256 && HD % 4 == 0 && LMAX > 0,
-              MIQ_ERR_INVALID, "attention: T=%d NH=%d NKV=%d HD=%d LMAX=%d", T, NH, NKV, HD, LMAX);
-  if (T == 0) return MIQ_OK;
-  MIQ_REQUIRE((size_t)LMAX * 4 <= 64 * 1024, MIQ_ERR_UNSUPPORTED, "attention: LMAX=%d above 16384", LMAX);
-  MIQ_REQUIRE(q && kcache && vcache && state && out, MIQ_ERR_INVALID, "attention: null pointer");
-  MIQ_REQUIRE(aligned(kcache, 16) && aligned(vcache, 16), MIQ_ERR_ALIGN, "attention: caches must be 16-byte aligned");
-  hipLaunchKernelGGL(attention_kernel, dim3(NH, T), dim3(64), (size_t)LMAX * 4, static_cast<hipStream_t>(stream), q,
-                     kcache, vcache, state, out, NH, NKV, HD, LMAX, scale);
-  return check_launch("attention");
 }
 
 extern "C" int miq_silu_mul(const float* gu, float* out, int T, int I, void* stream) {
