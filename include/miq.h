@@ -213,6 +213,15 @@ int miq_ggml_gemm_workspace(int M, int K, int N, int x_dtype, int ggml_type, siz
 int miq_ggml_gemm(const void* x, int x_dtype, const uint8_t* w, int ggml_type, const float* bias, void* out,
                   int out_dtype, int M, int K, int N, void* workspace, size_t ws_bytes, void* stream);
 
+/* miq_ggml_gemm for the 32-value nibble types 2 Q4_0, 6 Q5_0 and 20 IQ4_NL (8 consecutive blocks
+ * per 256-value step, every code an exact fp16 integer, d applied per block), with the same
+ * limits, alignments and workspace layout. Other types: MIQ_ERR_UNSUPPORTED.
+ * Replaces: `ggml_matmul` / `_ggml_run` for more than a few rows of these types
+ * (webtorch/_core.py:3720-3779; decoders `_Q4_0_DEC`, `_Q5_0_DEC` 3419-3468, `_IQ4NL_DEC` 3080). */
+int miq_ggml_nibble_gemm_workspace(int M, int K, int N, int x_dtype, int ggml_type, size_t* bytes);
+int miq_ggml_nibble_gemm(const void* x, int x_dtype, const uint8_t* w, int ggml_type, const float* bias, void* out,
+                         int out_dtype, int M, int K, int N, void* workspace, size_t ws_bytes, void* stream);
+
 /* out[M][N] = x[M][K] @ W^T + bias for the native GGUF types, by ggml type id:
  *   32-value blocks: 2 Q4_0, 3 Q4_1, 6 Q5_0, 7 Q5_1, 8 Q8_0, 20 IQ4_NL (18, 20, 22, 24, 34, 18
  *     bytes), 39 MXFP4 (17);

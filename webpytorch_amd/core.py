@@ -127,6 +127,13 @@ def workspace(nbytes):
     return t
 
 
+def workspace_holds(nbytes):
+    """Whether the current stream's workspace already has nbytes."""
+    dev = torch.cuda.current_device()
+    t = _WORKSPACE.get((dev, torch.cuda.current_stream(dev).cuda_stream))
+    return t is not None and t.numel() >= nbytes
+
+
 def aligned16(t):
     """The kernels read activations with 16-byte loads: copy a misaligned view."""
     return t if t.data_ptr() % 16 == 0 else t.clone()
@@ -456,13 +463,15 @@ def rows_from_transposed(words, n, rowb):
     return rows[:, :rowb].contiguous()
 
 
-# Q4_K rows above this count go to the matrix-core GEMM (the other types stay on the GEMV)
+# Rows above this count go to the matrix-core GEMM (types without one stay on the GEMV)
 GGML_GEMV_MAX_M = 8
 
 
 # Types whose rows above GGML_GEMV_MAX_M run on the matrix cores (`miq_ggml_gemm`), for K a
 # multiple of 256: the four types of a Q4_K_M / Q5_K_M file
 GGML_GEMM_TYPES = ("Q4_K", "Q5_K", "Q6_K", "Q8_0")
+# Types whose rows take `miq_ggml_nibble_gemm` where `_nibble_gemm_taken` says so
+GGML_NIBBLE_TYPES = ("Q4_0", "Q5_0", "IQ4_NL")
 
 
 def ggml_gemm_workspace_bytes(M, K, N, x_dtype, type_name="Q4_K"):
@@ -470,7 +479,8 @@ def ggml_gemm_workspace_bytes(M, K, N, x_dtype, type_name="Q4_K"):
     b = _WS_BYTES.get(key)
     if b is None:
         n = ctypes.c_size_t(0)
-        _lib.call("miq_ggml_gemm_workspace", M, K, N, x_dtype, _NATIVE_TYPES[type_name][2], ctypes.byref(n))
+        f = "miq_ggml_nibble_gemm_workspace" if type_name in GGML_NIBBLE_TYPES else "miq_ggml_gemm_workspace"
+        _lib.call(f, M, K, N, x_dtype, _NATIVE_TYPES[type_name][2], ctypes.byref(n))
         b = _WS_BYTES[key] = int(n.value)
     return b
 
@@ -481,6 +491,20 @@ def q4k_gemm_workspace_bytes(M, K, N, x_dtype):
 
 def _ggml_gemm_taken(type_name, M, K):
     return type_name in GGML_GEMM_TYPES and M > GGML_GEMV_MAX_M and K % 256 == 0
+
+
+def _nibble_gemm_taken(type_name, M, K, N, x_dtype, packed):
+    """Whether M rows of a nibble type run on the matrix cores; if not, the GEMV takes them. The
+    GEMM reads whole 256-value steps of 16-byte aligned rows, stages rows of up to 16384 values,
+    and keeps its scratch in the stream's workspace, which must not grow inside a graph capture
+    (the GEMV needs none). The GEMV's time grows with M K N and the GEMM's launches cost 26 us a
+    call: they meet near 2^28 (Q4_0, us a call, GEMM / GEMV: 4096 -> 4096 26 / 22 at 9 rows, 26 / 26
+    at 12, 26 / 33 at 16; 1024 -> 1024 26 / 18 at 33; 14336 -> 4096 40 / 97 at 9)."""
+    if not (type_name in GGML_NIBBLE_TYPES and GGML_GEMV_MAX_M < M <= 65535 and M * K * N >= 1 << 28
+            and K % 256 == 0 and K <= 16384 and packed.data_ptr() % 16 == 0):
+        return False
+    return (not torch.cuda.is_current_stream_capturing()
+            or workspace_holds(ggml_gemm_workspace_bytes(M, K, N, x_dtype, type_name)))
 
 
 def _ggml_selfcheck(type_name, mode):
@@ -527,7 +551,8 @@ def ggml_matmul(xf, packed, type_name, K, N, bias=None, out_dtype=torch.float32,
                                                                            int(N) * rowb))
     xf = aligned16(as_activation(xf).contiguous())
     M = int(xf.shape[0])
-    gemm = _ggml_gemm_taken(type_name, M, int(K))
+    nibble = _nibble_gemm_taken(type_name, M, int(K), int(N), dtype_code(xf), packed)
+    gemm = nibble or _ggml_gemm_taken(type_name, M, int(K))
     mode = -1 if gemm else (M if M <= 2 else 0)
     if _check and M and _first_use(("ggml", type_name, mode)):
         _ggml_selfcheck(type_name, mode)
@@ -536,8 +561,9 @@ def ggml_matmul(xf, packed, type_name, K, N, bias=None, out_dtype=torch.float32,
     if gemm:  # prefill rows on the matrix cores
         need = ggml_gemm_workspace_bytes(M, int(K), int(N), dtype_code(xf), type_name)
         ws = workspace(need)
-        _lib.call("miq_ggml_gemm", ptr(xf), dtype_code(xf), ptr(packed), _NATIVE_TYPES[type_name][2], ptr(bias),
-                  ptr(out), dtype_code(out), M, int(K), int(N), ptr(ws), ws.numel(), stream_handle())
+        _lib.call("miq_ggml_nibble_gemm" if nibble else "miq_ggml_gemm", ptr(xf), dtype_code(xf), ptr(packed),
+                  _NATIVE_TYPES[type_name][2], ptr(bias), ptr(out), dtype_code(out), M, int(K), int(N), ptr(ws),
+                  ws.numel(), stream_handle())
     elif type_name == "Q4_K":
         _lib.call("miq_q4k_gemv", ptr(xf), dtype_code(xf), ptr(packed), ptr(bias), ptr(out), dtype_code(out),
                   M, int(K), int(N), stream_handle())

@@ -1,14 +1,17 @@
-// GGUF K-quant prefill GEMM on the gfx950 matrix cores: out[m][n] = x[m][:] . W[n][:] (+ bias[n])
+// GGUF prefill GEMM on the gfx950 matrix cores: out[m][n] = x[m][:] . W[n][:] (+ bias[n])
 // for many activation rows, W = N rows of blocks as the file stores them, for the four types of
-// a Q4_K_M / Q5_K_M file: Q4_K, Q5_K, Q6_K and Q8_0 (8 consecutive 32-value blocks make one
-// 256-value step). Block layouts (llama.cpp's):
+// a Q4_K_M / Q5_K_M file (Q4_K, Q5_K, Q6_K and Q8_0) and the 32-value nibble types Q4_0, Q5_0
+// and IQ4_NL (8 consecutive 32-value blocks make one 256-value step). Block layouts (llama.cpp's):
 //   Q4_K (144 bytes): fp16 d, fp16 dmin, 12 bytes of 6-bit scales/mins, qs[128];
 //   Q5_K (176 bytes): the same header, qh[32], qs[128] -- the fifth bit of value l of
 //     sub-block j is bit j of qh[l];
 //   Q6_K (210 bytes): ql[128], qh[64], 16 int8 scales, fp16 d -- value 128 h + 32 j + l has code
 //     ((ql[64 h + 32 (j & 1) + l] >> 4 (j >> 1)) & 15) | ((qh[32 h + l] >> 2 j) & 3) << 4 and
 //     scale byte 8 h + 2 j + l / 16;
-//   Q8_0 (34 bytes): fp16 d, 32 int8 codes.
+//   Q8_0 (34 bytes): fp16 d, 32 int8 codes;
+//   Q4_0, IQ4_NL (18 bytes): fp16 d, qs[16] -- byte j holds the codes of values j (low nibble) and
+//     16 + j (high); w = d (c - 8), or d times entry c of a table of 16 int8 values;
+//   Q5_0 (22 bytes): fp16 d, a dword whose bit i is the fifth bit of value i, qs[16]; d (c - 16).
 //
 // Every product runs on the fp16 matrix cores with an exact integer B operand:
 //   * Q4_K / Q5_K: a sub-block of 32 weights holds w = d sc c - dmin m, so per sub-block
@@ -22,6 +25,11 @@
 //     d applies once per super-block.
 //   * Q8_0: B = q (int8, exact); each 32-value block has its own d, so every block's product
 //     starts from zero and is folded into the accumulator as d P (four fp32 FMAs per tile).
+//   * Q4_0, Q5_0, IQ4_NL: B = c - 8, c - 16 or the table value, folded block by block like Q8_0,
+//     but into a sum of the step's own that is added to the accumulator: a chain of K / 32
+//     roundings stood at 2.0e-7 from float64 at K = 4096, above the GEMV's 1.6e-7 (the GEMV, which
+//     takes few rows of these types, decodes the whole matrix once per row of x).
+//     Q4_0 4096 -> 4096, 77 fp32 rows: 139 us in the GEMV, 50 us here; 1.1e-7 from float64.
 // Codes become fp16 operands by OR-ing them into the mantissa of 1024.0 and subtracting 1024
 // (plus the code offset), no conversion instruction per code.
 //
@@ -87,7 +95,11 @@ __device__ __forceinline__ float sum8(const __half* h) {
 // fp16) with their sub-block sums, and for fp32 the row's largest |x| (NaN if it holds one) in
 // rmax[m]. The four threads of a sub-block are consecutive (quad), so its sum is a quad sum.
 // Dynamic LDS K * 4 bytes for fp32 (the row is read once, its maximum sets the scale).
-template <typename XT>
+//
+// NIB: the layout of the nibble types, whose code byte j of a 32-value block holds values j (low)
+// and 16 + j (high): chunk kb of a block holds values 4 kb .. + 3 and 16 + 4 kb .. + 3, so that a
+// lane's B operand is both nibbles of one dword.
+template <typename XT, bool NIB>
 __global__ __launch_bounds__(256) void stage_kernel(const XT* __restrict__ x, __half* __restrict__ xs,
                                                     float* __restrict__ rs, float* __restrict__ rmax, int K) {
   constexpr bool F32 = std::is_same<XT, float>::value;
@@ -125,12 +137,19 @@ __global__ __launch_bounds__(256) void stage_kernel(const XT* __restrict__ x, __
     if constexpr (F32) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float a = frow[8 * i + j] * sc;
+        const float a = frow[NIB ? 32 * (i >> 2) + 4 * (i & 3) + (j & 3) + 16 * (j >> 2) : 8 * i + j] * sc;
         hi[j] = __float2half_rn(a);
         lo[j] = __float2half_rn(a - __half2float(hi[j]));
       }
     } else {
-      const uint4 v = *reinterpret_cast<const uint4*>(x + (size_t)m * K + 8 * i);
+      uint4 v;
+      if constexpr (NIB) {
+        const uint2* b = reinterpret_cast<const uint2*>(x + (size_t)m * K + 32 * (i >> 2));
+        const uint2 lo4 = b[i & 3], hi4 = b[4 + (i & 3)];
+        v = make_uint4(lo4.x, lo4.y, hi4.x, hi4.y);
+      } else {
+        v = *reinterpret_cast<const uint4*>(x + (size_t)m * K + 8 * i);
+      }
       const uint32_t wv[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -150,8 +169,10 @@ __global__ __launch_bounds__(256) void stage_kernel(const XT* __restrict__ x, __
   }
 }
 
-// ggml type ids of the four types
+// ggml type ids
 constexpr int kQ8_0 = 8, kQ4_K = 12, kQ5_K = 13, kQ6_K = 14;
+constexpr int kQ4_0 = 2, kQ5_0 = 6, kIQ4_NL = 20;  // the nibble types
+constexpr bool is_nib(int t) { return t == kQ4_0 || t == kQ5_0 || t == kIQ4_NL; }
 
 // Per type: bytes per 256-value step, raw 32-bit registers per lane and step, whether the
 // sub-block mins (and so the row sums) enter.
@@ -160,6 +181,9 @@ template <> struct KQ<kQ4_K> { static constexpr int STEP = 144, RAW = 12; static
 template <> struct KQ<kQ5_K> { static constexpr int STEP = 176, RAW = 14; static constexpr bool MIN = true; };
 template <> struct KQ<kQ6_K> { static constexpr int STEP = 210, RAW = 24; static constexpr bool MIN = false; };
 template <> struct KQ<kQ8_0> { static constexpr int STEP = 272, RAW = 32; static constexpr bool MIN = false; };
+template <> struct KQ<kQ4_0> { static constexpr int STEP = 144, RAW = 20; static constexpr bool MIN = false; };
+template <> struct KQ<kIQ4_NL> { static constexpr int STEP = 144, RAW = 20; static constexpr bool MIN = false; };
+template <> struct KQ<kQ5_0> { static constexpr int STEP = 176, RAW = 28; static constexpr bool MIN = false; };
 
 __device__ __forceinline__ uint32_t ld32(const uint8_t* p) { return *reinterpret_cast<const uint32_t*>(p); }
 __device__ __forceinline__ uint32_t ld16(const uint8_t* p) { return *reinterpret_cast<const unsigned short*>(p); }
@@ -180,6 +204,14 @@ __device__ __forceinline__ uint32_t ld16(const uint8_t* p) { return *reinterpret
 //         codes for kb sit at a = 34 b + 2 + 8 kb, 4-byte aligned for odd b (two dwords) and
 //         2-byte aligned for even b (dwords at a - 2 and a + 2 and the 2 bytes at a + 6, ending
 //         at the block's last code byte); d of block b (fp16 at 34 b) in r[4b + 3].
+//   Q4_0, IQ4_NL: bp is 16-byte aligned (144-byte steps); the lane's code bytes of block b are
+//         the dword at a = 18 b + 2 + 4 kb: 4-byte aligned for odd b, else dwords at a - 2 and
+//         a + 2 (the second ends at most in the scale of block b + 1, which an even b has within
+//         the step). Blocks 2h and 2h + 1 in r[5h..]: the two dwords, d, the dword, d.
+//   Q5_0: bp is 16-byte aligned (176-byte steps); fifth bits (dword) at 22 b + 2, code bytes at
+//         a = 22 b + 6 + 4 kb, both 4-byte aligned for odd b; for even b d and the fifth bits are
+//         the dwords at 22 b and 22 b + 4, the codes dwords at a - 2 and a + 2 (again at most in
+//         block b + 1). Blocks 2h and 2h + 1 in r[7h..]: four dwords, then d, fifth bits, codes.
 template <int T> __device__ __forceinline__ void load_raw(const uint8_t* bp, int kb, uint32_t* r) {
   if constexpr (T == kQ4_K || T == kQ5_K) {
     const uint4 h = *reinterpret_cast<const uint4*>(bp);
@@ -213,6 +245,21 @@ template <int T> __device__ __forceinline__ void load_raw(const uint8_t* bp, int
     for (int i = 0; i < 4; ++i) r[18 + i] = ld32(b4 + 192 + 4 * i);
     r[22] = ld32(b4 + (s ? 208 : 204));
     r[23] = ld16(bp + 208);
+  } else if constexpr (T == kQ4_0 || T == kIQ4_NL) {
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const uint8_t* q = bp + 36 * h;
+      r[5 * h] = ld32(q + 4 * kb); r[5 * h + 1] = ld32(q + 4 * kb + 4); r[5 * h + 2] = ld16(q);
+      r[5 * h + 3] = ld32(q + 20 + 4 * kb); r[5 * h + 4] = ld16(q + 18);
+    }
+  } else if constexpr (T == kQ5_0) {
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const uint8_t* q = bp + 44 * h;
+      r[7 * h] = ld32(q); r[7 * h + 1] = ld32(q + 4);
+      r[7 * h + 2] = ld32(q + 4 + 4 * kb); r[7 * h + 3] = ld32(q + 8 + 4 * kb);
+      r[7 * h + 4] = ld16(q + 22); r[7 * h + 5] = ld32(q + 24); r[7 * h + 6] = ld32(q + 28 + 4 * kb);
+    }
   } else {
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
@@ -253,6 +300,17 @@ __device__ __forceinline__ half8v b_codes(uint32_t w0, uint32_t w1, _Float16 off
   const half2v d = as_h2(and_or(w1 >> 8, m, 0x64006400u)) - k;
   return (half8v){a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
+
+// IQ4_NL values + 128, four to a word: entries 0-3, 4-7, 8-11, 12-15
+constexpr uint32_t kNL[4] = {0x3F2D1801u, 0x766A5D4Fu, 0xA6998D81u, 0xF1D9C5B5u};
+// the table entries (+ 128) of the four 4-bit codes in the low nibbles of c's bytes
+__device__ __forceinline__ uint32_t nl_lookup(uint32_t c) {
+  const uint32_t s = c & 0x07070707u;
+  const uint32_t lo = __builtin_amdgcn_perm(kNL[1], kNL[0], s), hi = __builtin_amdgcn_perm(kNL[3], kNL[2], s);
+  return __builtin_amdgcn_perm(hi, lo, ((c & 0x08080808u) >> 1) | 0x03020100u);
+}
+// bits 0-3 of n as bit 4 of bytes 0-3 (n < 16: four copies of n, 7 bits apart, do not meet)
+__device__ __forceinline__ uint32_t spread4(uint32_t n) { return (__umul24(n, 0x204081u) & 0x01010101u) << 4; }
 
 __device__ __forceinline__ float f16f(uint32_t u) { return __half2float(__ushort_as_half((unsigned short)(u & 0xFFFFu))); }
 
@@ -450,18 +508,36 @@ __global__ __launch_bounds__(256) void gemm_kernel(const __half* __restrict__ xs
 #pragma unroll
           for (int q = 0; q < 4; ++q) acc[c][t][q] = fmaf(d, P[c][t][q], acc[c][t][q]);
       }
-    } else {  // Q8_0: one block per 32-value sub-block, its product folded with its own d
+    } else {  // one 32-value block per MFMA step, its product folded with its own d
+      constexpr bool NIB = is_nib(T);
+      float4v S[NIB ? CG : 1][4];  // the step's own sum
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
         half8v bf[CG];
         float d[CG];
 #pragma unroll
         for (int c = 0; c < CG; ++c) {
-          const uint32_t* R = raw[c] + 4 * b;
-          const uint32_t q0 = (b & 1) ? R[0] : __builtin_amdgcn_alignbyte(R[1], R[0], 2);
-          const uint32_t q1 = (b & 1) ? R[1] : __builtin_amdgcn_alignbyte(R[2], R[1], 2);
-          bf[c] = b_codes<0xFFu>(q0 ^ 0x80808080u, q1 ^ 0x80808080u, (_Float16)128);  // q, exact
-          d[c] = f16f(R[3]);
+          if constexpr (T == kQ8_0) {
+            const uint32_t* R = raw[c] + 4 * b;
+            const uint32_t q0 = (b & 1) ? R[0] : __builtin_amdgcn_alignbyte(R[1], R[0], 2);
+            const uint32_t q1 = (b & 1) ? R[1] : __builtin_amdgcn_alignbyte(R[2], R[1], 2);
+            bf[c] = b_codes<0xFFu>(q0 ^ 0x80808080u, q1 ^ 0x80808080u, (_Float16)128);  // q, exact
+            d[c] = f16f(R[3]);
+          } else if constexpr (T == kQ5_0) {
+            const uint32_t* R = raw[c] + 7 * (b >> 1);
+            const uint32_t q = (b & 1) ? R[6] : __builtin_amdgcn_alignbyte(R[3], R[2], 2);
+            const uint32_t qh = ((b & 1) ? R[5] : __builtin_amdgcn_alignbyte(R[1], R[0], 2)) >> (4 * kb);
+            d[c] = f16f((b & 1) ? R[4] : R[0]);
+            const uint32_t c0 = (q & 0x0F0F0F0Fu) | spread4(qh & 15u);
+            const uint32_t c1 = ((q >> 4) & 0x0F0F0F0Fu) | spread4((qh >> 16) & 15u);
+            bf[c] = b_codes<0x1Fu>(c0, c1, (_Float16)16);  // q - 16, exact
+          } else {
+            const uint32_t* R = raw[c] + 5 * (b >> 1);
+            const uint32_t q = (b & 1) ? R[3] : __builtin_amdgcn_alignbyte(R[1], R[0], 2);
+            d[c] = f16f((b & 1) ? R[4] : R[2]);
+            if constexpr (T == kQ4_0) bf[c] = b_codes<0x0Fu>(q, q >> 4, (_Float16)8);  // q - 8, exact
+            else bf[c] = b_codes<0xFFu>(nl_lookup(q), nl_lookup(q >> 4), (_Float16)128);  // table value, exact
+          }
         }
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -470,9 +546,18 @@ __global__ __launch_bounds__(256) void gemm_kernel(const __half* __restrict__ xs
           for (int c = 0; c < CG; ++c) {
             const float4v P = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[c], (float4v){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc[c][t][q] = fmaf(d[c], P[q], acc[c][t][q]);
+            for (int q = 0; q < 4; ++q) {
+              if constexpr (NIB) S[c][t][q] = b ? fmaf(d[c], P[q], S[c][t][q]) : d[c] * P[q];
+              else acc[c][t][q] = fmaf(d[c], P[q], acc[c][t][q]);
+            }
           }
         }
+      }
+      if constexpr (NIB) {
+#pragma unroll
+        for (int c = 0; c < CG; ++c)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) acc[c][t] += S[c][t];
       }
     }
   }
@@ -609,61 +694,91 @@ static int gemm_t(const __half* xs, const float* rs, const float* rmax, float* p
   return go(static_cast<float*>(out), std::true_type{});
 }
 
-}  // namespace kg
-}  // namespace miq
-
-using namespace miq;
-
-extern "C" int miq_ggml_gemm_workspace(int M, int K, int N, int x_dtype, int ggml_type, size_t* bytes) {
-  MIQ_REQUIRE(bytes, MIQ_ERR_INVALID, "ggml_gemm_workspace: null output");
-  MIQ_REQUIRE(kg::covered(ggml_type), MIQ_ERR_UNSUPPORTED, "ggml_gemm_workspace: ggml type %d has no GEMM",
-              ggml_type);
-  MIQ_REQUIRE(M >= 0 && K > 0 && N > 0 && K % 256 == 0, MIQ_ERR_INVALID, "ggml_gemm_workspace: M=%d K=%d N=%d", M, K,
-              N);
-  MIQ_REQUIRE(x_dtype == MIQ_F16 || x_dtype == MIQ_F32, MIQ_ERR_UNSUPPORTED, "ggml_gemm_workspace: x dtype");
-  *bytes = M == 0 ? 0 : kg::layout(M, K, N, x_dtype).bytes;
+static int workspace_call(const char* who, bool ok, int M, int K, int N, int x_dtype, int ggml_type, size_t* bytes) {
+  MIQ_REQUIRE(bytes, MIQ_ERR_INVALID, "%s: null output", who);
+  MIQ_REQUIRE(ok, MIQ_ERR_UNSUPPORTED, "%s: ggml type %d has no GEMM", who, ggml_type);
+  MIQ_REQUIRE(M >= 0 && K > 0 && N > 0 && K % 256 == 0, MIQ_ERR_INVALID, "%s: M=%d K=%d N=%d", who, M, K, N);
+  MIQ_REQUIRE(x_dtype == MIQ_F16 || x_dtype == MIQ_F32, MIQ_ERR_UNSUPPORTED, "%s: x dtype", who);
+  *bytes = M == 0 ? 0 : layout(M, K, N, x_dtype).bytes;
   return MIQ_OK;
 }
 
-extern "C" int miq_ggml_gemm(const void* x, int x_dtype, const uint8_t* w, int ggml_type, const float* bias, void* out,
-                             int out_dtype, int M, int K, int N, void* workspace, size_t ws_bytes, void* stream) {
-  MIQ_REQUIRE(kg::covered(ggml_type), MIQ_ERR_UNSUPPORTED, "ggml_gemm: ggml type %d has no GEMM", ggml_type);
-  MIQ_REQUIRE(M >= 0 && K > 0 && N > 0, MIQ_ERR_INVALID, "ggml_gemm: M=%d K=%d N=%d", M, K, N);
-  MIQ_REQUIRE(K % 256 == 0, MIQ_ERR_INVALID, "ggml_gemm: K=%d is not a multiple of 256", K);
-  MIQ_REQUIRE(x_dtype == MIQ_F16 || x_dtype == MIQ_F32, MIQ_ERR_UNSUPPORTED, "ggml_gemm: x dtype");
-  MIQ_REQUIRE(out_dtype == MIQ_F16 || out_dtype == MIQ_F32, MIQ_ERR_UNSUPPORTED, "ggml_gemm: out dtype");
+template <bool NIB>
+static int stage(const void* x, int x_dtype, __half* xs, float* rs, float* rmax, int M, int K, hipStream_t st) {
+  if (x_dtype == MIQ_F32) {
+    if ((size_t)K * 4 > 64 * 1024) {
+      const int rc = require_lds("ggml_gemm staging", (size_t)K * 4);
+      if (rc) return rc;
+    }
+    hipLaunchKernelGGL((stage_kernel<float, NIB>), dim3(M), dim3(256), (size_t)K * 4, st, static_cast<const float*>(x),
+                       xs, rs, rmax, K);
+  } else {
+    hipLaunchKernelGGL((stage_kernel<__half, NIB>), dim3(M), dim3(256), 0, st, static_cast<const __half*>(x), xs, rs,
+                       rmax, K);
+  }
+  return check_launch("ggml_gemm staging");
+}
+
+static int gemm_call(const char* who, bool ok, const void* x, int x_dtype, const uint8_t* w, int ggml_type,
+                     const float* bias, void* out, int out_dtype, int M, int K, int N, void* workspace,
+                     size_t ws_bytes, void* stream) {
+  MIQ_REQUIRE(ok, MIQ_ERR_UNSUPPORTED, "%s: ggml type %d has no GEMM", who, ggml_type);
+  MIQ_REQUIRE(M >= 0 && K > 0 && N > 0, MIQ_ERR_INVALID, "%s: M=%d K=%d N=%d", who, M, K, N);
+  MIQ_REQUIRE(K % 256 == 0, MIQ_ERR_INVALID, "%s: K=%d is not a multiple of 256", who, K);
+  MIQ_REQUIRE(x_dtype == MIQ_F16 || x_dtype == MIQ_F32, MIQ_ERR_UNSUPPORTED, "%s: x dtype", who);
+  MIQ_REQUIRE(out_dtype == MIQ_F16 || out_dtype == MIQ_F32, MIQ_ERR_UNSUPPORTED, "%s: out dtype", who);
   if (M == 0) return MIQ_OK;
-  MIQ_REQUIRE(x && w && out && workspace, MIQ_ERR_INVALID, "ggml_gemm: null pointer");
+  MIQ_REQUIRE(x && w && out && workspace, MIQ_ERR_INVALID, "%s: null pointer", who);
   MIQ_REQUIRE(aligned(w, 16) && aligned(x, 16) && aligned(workspace, 256), MIQ_ERR_ALIGN,
-              "ggml_gemm: x and weight 16-byte, workspace 256-byte aligned");
-  const kg::Ws L = kg::layout(M, K, N, x_dtype);
-  MIQ_REQUIRE(ws_bytes >= L.bytes, MIQ_ERR_INVALID, "ggml_gemm: workspace %zu bytes, need %zu", ws_bytes, L.bytes);
-  MIQ_REQUIRE(K <= 16384, MIQ_ERR_UNSUPPORTED, "ggml_gemm: K=%d too large to stage", K);
+              "%s: x and weight 16-byte, workspace 256-byte aligned", who);
+  const Ws L = layout(M, K, N, x_dtype);
+  MIQ_REQUIRE(ws_bytes >= L.bytes, MIQ_ERR_INVALID, "%s: workspace %zu bytes, need %zu", who, ws_bytes, L.bytes);
+  MIQ_REQUIRE(K <= 16384, MIQ_ERR_UNSUPPORTED, "%s: K=%d too large to stage", who, K);
   hipStream_t st = static_cast<hipStream_t>(stream);
   unsigned char* b = static_cast<unsigned char*>(workspace);
   __half* xs = reinterpret_cast<__half*>(b + L.xs);
   float* rs = reinterpret_cast<float*>(b + L.rs);
   float* rmax = reinterpret_cast<float*>(b + L.rmax);
   float* part = reinterpret_cast<float*>(b + L.part);
-  if (x_dtype == MIQ_F32) {
-    if ((size_t)K * 4 > 64 * 1024) {
-      const int rc = require_lds("ggml_gemm staging", (size_t)K * 4);
-      if (rc) return rc;
-    }
-    hipLaunchKernelGGL(kg::stage_kernel<float>, dim3(M), dim3(256), (size_t)K * 4, st, static_cast<const float*>(x), xs,
-                       rs, rmax, K);
-  } else {
-    hipLaunchKernelGGL(kg::stage_kernel<__half>, dim3(M), dim3(256), 0, st, static_cast<const __half*>(x), xs, rs, rmax,
-                       K);
-  }
-  const int rc = check_launch("ggml_gemm staging");
+  const int rc = is_nib(ggml_type) ? stage<true>(x, x_dtype, xs, rs, rmax, M, K, st)
+                                   : stage<false>(x, x_dtype, xs, rs, rmax, M, K, st);
   if (rc) return rc;
   switch (ggml_type) {
-    case kg::kQ4_K: return kg::gemm_t<kg::kQ4_K>(xs, rs, rmax, part, w, bias, out, out_dtype, M, x_dtype, K, N, st);
-    case kg::kQ5_K: return kg::gemm_t<kg::kQ5_K>(xs, rs, rmax, part, w, bias, out, out_dtype, M, x_dtype, K, N, st);
-    case kg::kQ6_K: return kg::gemm_t<kg::kQ6_K>(xs, rs, rmax, part, w, bias, out, out_dtype, M, x_dtype, K, N, st);
-    default: return kg::gemm_t<kg::kQ8_0>(xs, rs, rmax, part, w, bias, out, out_dtype, M, x_dtype, K, N, st);
+    case kQ4_K: return gemm_t<kQ4_K>(xs, rs, rmax, part, w, bias, out, out_dtype, M, x_dtype, K, N, st);
+    case kQ5_K: return gemm_t<kQ5_K>(xs, rs, rmax, part, w, bias, out, out_dtype, M, x_dtype, K, N, st);
+    case kQ6_K: return gemm_t<kQ6_K>(xs, rs, rmax, part, w, bias, out, out_dtype, M, x_dtype, K, N, st);
+    case kQ4_0: return gemm_t<kQ4_0>(xs, rs, rmax, part, w, bias, out, out_dtype, M, x_dtype, K, N, st);
+    case kQ5_0: return gemm_t<kQ5_0>(xs, rs, rmax, part, w, bias, out, out_dtype, M, x_dtype, K, N, st);
+    case kIQ4_NL: return gemm_t<kIQ4_NL>(xs, rs, rmax, part, w, bias, out, out_dtype, M, x_dtype, K, N, st);
+    default: return gemm_t<kQ8_0>(xs, rs, rmax, part, w, bias, out, out_dtype, M, x_dtype, K, N, st);
   }
+}
+
+}  // namespace kg
+}  // namespace miq
+
+using namespace miq;
+
+extern "C" int miq_ggml_gemm_workspace(int M, int K, int N, int x_dtype, int ggml_type, size_t* bytes) {
+  return kg::workspace_call("ggml_gemm_workspace", kg::covered(ggml_type), M, K, N, x_dtype, ggml_type, bytes);
+}
+
+extern "C" int miq_ggml_gemm(const void* x, int x_dtype, const uint8_t* w, int ggml_type, const float* bias, void* out,
+                             int out_dtype, int M, int K, int N, void* workspace, size_t ws_bytes, void* stream) {
+  return kg::gemm_call("ggml_gemm", kg::covered(ggml_type), x, x_dtype, w, ggml_type, bias, out, out_dtype, M, K, N,
+                       workspace, ws_bytes, stream);
+}
+
+extern "C" int miq_ggml_nibble_gemm_workspace(int M, int K, int N, int x_dtype, int ggml_type, size_t* bytes) {
+  return kg::workspace_call("ggml_nibble_gemm_workspace", kg::is_nib(ggml_type), M, K, N, x_dtype, ggml_type,
+                            bytes);
+}
+
+extern "C" int miq_ggml_nibble_gemm(const void* x, int x_dtype, const uint8_t* w, int ggml_type, const float* bias,
+                                    void* out, int out_dtype, int M, int K, int N, void* workspace, size_t ws_bytes,
+                                    void* stream) {
+  return kg::gemm_call("ggml_nibble_gemm", kg::is_nib(ggml_type), x, x_dtype, w, ggml_type, bias, out, out_dtype,
+                       M, K, N, workspace, ws_bytes, stream);
 }
 
 extern "C" int miq_q4k_gemm_workspace(int M, int K, int N, int x_dtype, size_t* bytes) {
