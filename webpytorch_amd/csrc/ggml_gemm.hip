@@ -17,8 +17,14 @@
 //   * Q4_K / Q5_K: a sub-block of 32 weights holds w = d sc c - dmin m, so per sub-block
 //     sum_k x_k w_k = d (sc sum_k x_k c_k) - dmin (m sum_k x_k); B = sc c is an integer below
 //     2048 (63 x 31 at most), exact in fp16, so the eight sub-blocks chain in one accumulator;
-//     the row sums of x come precomputed per sub-block and the mins multiply them on the fp32
-//     matrix cores; d and dmin apply once per super-block.
+//     the row sums of x come precomputed per sub-block and the mins multiply them in one bf16
+//     MFMA per 16 x 16 tile and super-block (its 32 k slots are 8 sub-blocks x the 3 bf16 of a sum;
+//     the mins, below 64, are exact); d and dmin apply once per super-block. Before, two fp32
+//     MFMAs took the mins (a third of the matrix-core time) and every scale was cut out of its
+//     packed bytes on its own: 4096 -> 14336, 512 fp16 rows, 142 -> 108 us. What is left is the
+//     unpack (about 450 vector instructions against 72 MFMAs per wave and step) and the wait at
+//     each step's barrier with two waves a SIMD; tiles of 256 columns measured 5 % slower, loads
+//     spread over the sub-blocks no faster.
 //   * Q6_K: w = d sc (c - 32) with a signed 8-bit sc and 16-value sub-blocks, so (c - 32) sc
 //     (up to 4096) is not exact in fp16; sc = 16 sh + sl (sl = sc & 15, sh = sc >> 4) splits it
 //     into two exact operands, (c - 32) sl and (c - 32) 16 sh, two MFMAs into one accumulator;
@@ -41,7 +47,7 @@
 // Staged rows: xs[r][k] fp16, each 8-wide k block in the order (0, 2, 1, 3, 4, 6, 5, 7) that
 // the code unpack produces (byte j of a code word holds value j, and one v_and_or_b32 takes
 // bytes 0 and 2, then 1 and 3); rs[r][k / 32] the sub-block sums of the staged fp16 values
-// (fp32).
+// (fp32, held as three bf16 and a zero whose sum is the fp32 value exactly).
 //
 // Tiles: a workgroup of 4 waves computes 64 rows x 64 CG columns; wave w takes the CG groups of
 // 16 columns from 16 CG w and all 64 rows (four 16-row MFMA tiles per group). K is walked 256
@@ -70,6 +76,7 @@ constexpr int kCUs = 256;
 
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 typedef float float4v __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ int row_exp(float m) {
   if (!(m > 0.f) || !(m <= 3.4e38f)) return 0;
@@ -91,6 +98,17 @@ __device__ __forceinline__ float sum8(const __half* h) {
          ((__half2float(h[4]) + __half2float(h[5])) + (__half2float(h[6]) + __half2float(h[7])));
 }
 
+// v as three bf16 (top first) whose sum is v: truncations of 8 significant bits each, exact for
+// every normal v (the remainders are exact differences). A value that is not finite stays whole.
+__device__ __forceinline__ uint2 split_bf16(float v) {
+  const uint32_t h = __float_as_uint(v) & 0xFFFF0000u;
+  if ((h & 0x7F800000u) == 0x7F800000u) return make_uint2(h >> 16, 0u);
+  const float r = v - __uint_as_float(h);
+  const uint32_t m = __float_as_uint(r) & 0xFFFF0000u;
+  const float q = r - __uint_as_float(m);
+  return make_uint2((h >> 16) | m, __float_as_uint(q) >> 16);
+}
+
 // One workgroup per row m of x: rows R m .. R m + R - 1 of xs (R = 2 for fp32 x: hi, lo; 1 for
 // fp16) with their sub-block sums, and for fp32 the row's largest |x| (NaN if it holds one) in
 // rmax[m]. The four threads of a sub-block are consecutive (quad), so its sum is a quad sum.
@@ -101,7 +119,7 @@ __device__ __forceinline__ float sum8(const __half* h) {
 // lane's B operand is both nibbles of one dword.
 template <typename XT, bool NIB>
 __global__ __launch_bounds__(256) void stage_kernel(const XT* __restrict__ x, __half* __restrict__ xs,
-                                                    float* __restrict__ rs, float* __restrict__ rmax, int K) {
+                                                    uint2* __restrict__ rs, float* __restrict__ rmax, int K) {
   constexpr bool F32 = std::is_same<XT, float>::value;
   const int m = blockIdx.x, nch = K / 8, K32 = K / 32;
   float sc = 1.f;
@@ -160,11 +178,11 @@ __global__ __launch_bounds__(256) void stage_kernel(const XT* __restrict__ x, __
     constexpr int R = F32 ? 2 : 1;
     *reinterpret_cast<uint4*>(xs + ((size_t)R * m) * K + 8 * i) = order8(hi);
     const float shi = quad_sum(sum8(hi));
-    if ((i & 3) == 0) rs[((size_t)R * m) * K32 + i / 4] = shi;
+    if ((i & 3) == 0) rs[((size_t)R * m) * K32 + i / 4] = split_bf16(shi);
     if constexpr (F32) {
       *reinterpret_cast<uint4*>(xs + ((size_t)R * m + 1) * K + 8 * i) = order8(lo);
       const float slo = quad_sum(sum8(lo));
-      if ((i & 3) == 0) rs[((size_t)R * m + 1) * K32 + i / 4] = slo;
+      if ((i & 3) == 0) rs[((size_t)R * m + 1) * K32 + i / 4] = split_bf16(slo);
     }
   }
 }
@@ -274,18 +292,28 @@ template <int T> __device__ __forceinline__ void load_raw(const uint8_t* bp, int
   }
 }
 
-// The 6-bit scale and min of sub-block j from the 12 packed bytes (words s0, s1, s2 = bytes
-// 0-3, 4-7, 8-11).
-__device__ __forceinline__ void scale_min(uint32_t s0, uint32_t s1, uint32_t s2, int j, uint32_t* sc, uint32_t* mn) {
-  const uint32_t q[3] = {s0, s1, s2};
-  auto byte = [&](int b) { return (q[b >> 2] >> (8 * (b & 3))) & 0xFFu; };
-  if (j < 4) {
-    *sc = byte(j) & 63u;
-    *mn = byte(j + 4) & 63u;
-  } else {
-    *sc = (byte(j + 4) & 15u) | ((byte(j - 4) >> 6) << 4);
-    *mn = (byte(j + 4) >> 4) | ((byte(j) >> 6) << 4);
-  }
+// The 6-bit scales (sc) and mins (mn) of the 8 sub-blocks, one per byte, from the 12 packed bytes
+// (words s0, s1, s2 = bytes 0-3, 4-7, 8-11).
+__device__ __forceinline__ void scale_mins(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t* sc, uint32_t* mn) {
+  sc[0] = s0 & 0x3F3F3F3Fu;
+  mn[0] = s1 & 0x3F3F3F3Fu;
+  sc[1] = (s2 & 0x0F0F0F0Fu) | ((s0 >> 2) & 0x30303030u);
+  mn[1] = ((s2 >> 4) & 0x0F0F0F0Fu) | ((s1 >> 2) & 0x30303030u);
+}
+// byte j of w as an fp16 pair (both halves), by way of 1024 + byte
+__device__ __forceinline__ half2v byte_h2(uint32_t w, int j) {
+  const uint32_t v = __builtin_amdgcn_perm(w, 0x64646464u, (uint32_t)(4 + j) * 0x00010001u);
+  return as_h2(v) - (half2v){(_Float16)1024, (_Float16)1024};
+}
+// Four bytes of codes c in the bits of MASK of each byte (a nibble at bit 0 or 4) times an integer
+// scale, as two fp16 pairs (bytes 0, 2 and 1, 3): (1024 + c 2^k) s 2^-k - 1024 s 2^-k, one
+// rounding of an exact integer below 2048. w8 = w >> 8; s = scale 2^-k, off = -1024 s.
+template <uint32_t MASK> __device__ __forceinline__ half2v code_fma(uint32_t w, half2v s, half2v off) {
+  return __builtin_elementwise_fma(as_h2(and_or(w, MASK | (MASK << 16), 0x64006400u)), s, off);
+}
+// the bf16 of an integer below 256, twice
+__device__ __forceinline__ uint32_t bf16_pair(float f) {
+  return __builtin_amdgcn_perm(__float_as_uint(f), __float_as_uint(f), 0x03020302u);
 }
 
 // Codes in the low M bits of bytes 0-3 of w0 and 4-7 of w1 (the bits above masked off) as the
@@ -320,14 +348,14 @@ __device__ __forceinline__ float f16f(uint32_t u) { return __half2float(__ushort
 // (Q4_K / Q5_K) the row sums arrive by LDS DMA into one of two buffers while the other is
 // multiplied (the swizzle is applied on the source side: DMA lane l of a 1 KB block lands at
 // slot l); each lane's block bytes are loaded into registers one step ahead. Q4_K / Q5_K:
-// P = sum_sb sc_sb (x . c_sb) on the fp16 matrix cores, Q = sum_sb m_sb rs_sb on the fp32
-// matrix cores (two v_mfma_f32_16x16x4_f32: A the row sums, B the column's 6-bit mins), then
+// P = sum_sb sc_sb (x . c_sb) on the fp16 matrix cores, Q = sum_sb m_sb rs_sb on the bf16
+// matrix cores (A the row sums' three bf16, B the column's 6-bit mins), then
 // acc += d P - dmin Q. The output (+ bias[n]) as OT. fp16 rows (PAIR false): y[row][n] = acc.
 // fp32 rows (PAIR true): staged rows 2m and 2m + 1 are the hi and lo planes of row m, held by
 // the same lane (rows 4 kb + r of a 16-row tile), so y[m][n] = (acc[2m] + acc[2m + 1]) 2^-s(m),
 // s from rmax[m].
 template <int T, int CG, typename OT, bool PAIR>
-__global__ __launch_bounds__(256) void gemm_kernel(const __half* __restrict__ xs, const float* __restrict__ rs,
+__global__ __launch_bounds__(256, 2) void gemm_kernel(const __half* __restrict__ xs, const uint2* __restrict__ rs,
                                                    const uint8_t* __restrict__ w, OT* __restrict__ y,
                                                    const float* __restrict__ bias, const float* __restrict__ rmax,
                                                    int Mx, int K, int N, int mtiles, int tiles, int ksteps,
@@ -335,10 +363,9 @@ __global__ __launch_bounds__(256) void gemm_kernel(const __half* __restrict__ xs
   constexpr int RAW = KQ<T>::RAW, STEP = KQ<T>::STEP;
   constexpr bool MIN = KQ<T>::MIN;
   __shared__ __align__(16) __half at[2][kBM * 256];  // activation tiles, 16-byte chunks swizzled by row
-  // sub-block sums [sub-block][row], rows of kRT floats: the lanes of one read take rows p and
-  // sub-blocks kb, and at 64 floats (256 bytes) per sub-block the four kb share their banks
-  constexpr int kRT = kBM + 16;
-  __shared__ __align__(16) float rt[MIN ? 2 : 1][MIN ? 8 * kRT : 1];
+  // sub-block sums: 64 bytes a row, its 16-byte chunks (two sub-blocks each) swizzled by row / 4, so
+  // that 16 rows of one chunk fall in different banks
+  __shared__ __align__(16) uint2 rt[MIN ? 2 : 1][MIN ? kBM * 8 : 1];
   const int Tg = (int)gridDim.x, L = (int)blockIdx.x;
   const int Lp = Tg % kXCDs == 0 ? (L % kXCDs) * (Tg / kXCDs) + L / kXCDs : L;
   // K-slice kz of a split product (part != null): steps [s0, s1) of the row, raw sums to part
@@ -357,8 +384,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(const __half* __restrict__ xs
     wr[c] = w + (size_t)n * nsb * STEP;
   }
 
-  // this wave's share of the copies of step s into buffer b: 8 of the tile's 32 KB (two rows
-  // per 1 KB block) and 2 of its 8 sub-block-sum columns
+  // this wave's share of the copies of step s into buffer b: 8 of the tile's 32 KB (two rows per
+  // 1 KB block) and 1 of the 4 KB of sub-block sums
   auto issue = [&](int s, int b) __attribute__((always_inline)) {
     const uint32_t abase = lds_addr(at[b]);
 #pragma unroll
@@ -367,12 +394,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(const __half* __restrict__ xs
       dma16(xs + (size_t)min(m0 + r, Mx - 1) * K + s * 256 + c * 8, uniform((int)(abase + j * 1024)));
     }
     if constexpr (MIN) {
-      const uint32_t rbase = lds_addr(rt[b]);
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int sb = wave * 2 + i;
-        dma4(rs + (size_t)min(m0 + lane, Mx - 1) * K32 + s * 8 + sb, uniform((int)(rbase + sb * kRT * 4)));
-      }
+      const int r = 16 * wave + (lane >> 2), c = (lane & 3) ^ ((r >> 2) & 3);
+      dma16(rs + (size_t)min(m0 + r, Mx - 1) * K32 + s * 8 + 2 * c, uniform((int)(lds_addr(rt[b]) + wave * 1024)));
     }
   };
   uint32_t raw[CG][RAW], nxt[CG][RAW];
@@ -407,21 +430,34 @@ __global__ __launch_bounds__(256) void gemm_kernel(const __half* __restrict__ xs
 #pragma unroll
       for (int c = 0; c < CG; ++c)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) P[c][t] = Q[c][t] = (float4v){0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < 4; ++t) P[c][t] = (float4v){0.f, 0.f, 0.f, 0.f};
+      uint32_t sc[CG][2], mn[CG][2];
+#pragma unroll
+      for (int c = 0; c < CG; ++c) scale_mins(raw[c][1], raw[c][2], raw[c][3], sc[c], mn[c]);
 #pragma unroll
       for (int sb = 0; sb < 8; ++sb) {
-        const int sh = 4 * (sb & 1), g = sb >> 1;
+        const int g = sb >> 1;
         half8v bf[CG];
 #pragma unroll
         for (int c = 0; c < CG; ++c) {
-          uint32_t sc, mn;
-          scale_min(raw[c][1], raw[c][2], raw[c][3], sb, &sc, &mn);
-          uint32_t c0 = raw[c][4 + 2 * g] >> sh, c1 = raw[c][5 + 2 * g] >> sh;  // b_codes masks Q4_K's
-          if constexpr (T == kQ5_K) {
-            c0 = (c0 & 0x0F0F0F0Fu) | (((raw[c][12] >> sb) & 0x01010101u) << 4);
-            c1 = (c1 & 0x0F0F0F0Fu) | (((raw[c][13] >> sb) & 0x01010101u) << 4);
+          uint32_t c0 = raw[c][4 + 2 * g], c1 = raw[c][5 + 2 * g];
+          half2v s = byte_h2(sc[c][sb >> 2], sb & 3);
+          if (T == kQ4_K && (sb & 1)) {  // the high nibbles where they lie: 1024 + 16 c
+            s *= (half2v){(_Float16)0.0625f, (_Float16)0.0625f};
+            const half2v off = s * (half2v){(_Float16)-1024, (_Float16)-1024};
+            bf[c] = cat4(code_fma<0xF0u>(c0, s, off), code_fma<0xF0u>(c0 >> 8, s, off), code_fma<0xF0u>(c1, s, off),
+                         code_fma<0xF0u>(c1 >> 8, s, off));
+          } else {
+            if constexpr (T == kQ5_K) {
+              const int sh = 4 * (sb & 1);
+              c0 = ((c0 >> sh) & 0x0F0F0F0Fu) | (((raw[c][12] >> sb) & 0x01010101u) << 4);
+              c1 = ((c1 >> sh) & 0x0F0F0F0Fu) | (((raw[c][13] >> sb) & 0x01010101u) << 4);
+            }
+            constexpr uint32_t M = T == kQ5_K ? 0x1Fu : 0x0Fu;
+            const half2v off = s * (half2v){(_Float16)-1024, (_Float16)-1024};
+            bf[c] = cat4(code_fma<M>(c0, s, off), code_fma<M>(c0 >> 8, s, off), code_fma<M>(c1, s, off),
+                         code_fma<M>(c1 >> 8, s, off));
           }
-          bf[c] = b_codes<T == kQ5_K ? 0x1Fu : 0x0Fu>(c0, c1, (_Float16)0) * (_Float16)(float)sc;
         }
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -430,25 +466,23 @@ __global__ __launch_bounds__(256) void gemm_kernel(const __half* __restrict__ xs
           for (int c = 0; c < CG; ++c) P[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[c], P[c][t], 0, 0, 0);
         }
       }
-      {  // Q = sum over the 8 sub-blocks of rs[row][sb] m[sb][col]: k = kb, then 4 + kb
-        const float* r8 = rt[s & 1];
-        float m_lo[CG], m_hi[CG];
+      {  // Q = sum over the 8 sub-blocks of rs[row][sb] m[sb][col]; lane kb holds sub-blocks 2 kb, 2 kb + 1
+        bf16x8 bm[CG];
 #pragma unroll
         for (int c = 0; c < CG; ++c) {
-          uint32_t sc, mlo, mhi;
-          scale_min(raw[c][1], raw[c][2], raw[c][3], kb, &sc, &mlo);
-          scale_min(raw[c][1], raw[c][2], raw[c][3], 4 + kb, &sc, &mhi);
-          m_lo[c] = (float)mlo;
-          m_hi[c] = (float)mhi;
+          const uint32_t m2 = mn[c][1] & -(uint32_t)(kb >> 1) | mn[c][0] & ((uint32_t)(kb >> 1) - 1u);
+          const uint32_t mv = m2 >> (16 * (kb & 1));
+          const uint32_t lo = bf16_pair((float)(mv & 0xFFu)), hi = bf16_pair((float)((mv >> 8) & 0xFFu));
+          bm[c] = __builtin_bit_cast(bf16x8, make_uint4(lo, lo, hi, hi));
         }
+        const char* r8 = reinterpret_cast<const char*>(rt[s & 1]);
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const float rlo = r8[kb * kRT + 16 * t + p], rhi = r8[(4 + kb) * kRT + 16 * t + p];
+          const int r = 16 * t + p;
+          const bf16x8 ar = *reinterpret_cast<const bf16x8*>(r8 + r * 64 + ((kb ^ ((r >> 2) & 3)) * 16));
 #pragma unroll
-          for (int c = 0; c < CG; ++c) {
-            Q[c][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(rlo, m_lo[c], Q[c][t], 0, 0, 0);
-            Q[c][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(rhi, m_hi[c], Q[c][t], 0, 0, 0);
-          }
+          for (int c = 0; c < CG; ++c)
+            Q[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ar, bm[c], (float4v){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
         }
       }
 #pragma unroll
@@ -650,7 +684,7 @@ static Ws layout(int M, int K, int N, int x_dtype) {
   Ws w;
   w.xs = kCounterBytes;
   w.rs = w.xs + up(Mx * K * 2);
-  w.rmax = w.rs + up(Mx * (K / 32) * 4);
+  w.rmax = w.rs + up(Mx * (K / 32) * 8);
   w.part = w.rmax + up((size_t)M * 4);
   const Plan p = plan(M, K, N, x_dtype);
   w.bytes = w.part + (p.ksplit > 1 ? up((size_t)p.ksplit * Mx * N * 4) : 0);
@@ -661,10 +695,10 @@ static bool covered(int t) { return t == kQ4_K || t == kQ5_K || t == kQ6_K || t 
 
 // The GEMM of type T over staged rows. Two 16-column groups per wave (each activation operand
 // read feeds two MFMAs) when that grid still gives every CU two workgroups; otherwise one
-// (measured for Q4_K at 4096 -> 14336: fp32 rows at M = 512 288 -> 250 us, fp16 152 -> 149 us;
-// at M = 64 the halved grid was slower, 36 -> 51 us), and K split when even that grid is small.
+// (measured for Q4_K at 4096 -> 14336 when it was chosen: fp32 rows at M = 512 288 -> 250 us, fp16
+// 152 -> 149 us; at M = 64 the halved grid was slower, 36 -> 51 us), and K split when even that grid is small.
 template <int T>
-static int gemm_t(const __half* xs, const float* rs, const float* rmax, float* part, const uint8_t* w,
+static int gemm_t(const __half* xs, const uint2* rs, const float* rmax, float* part, const uint8_t* w,
                   const float* bias, void* out, int out_dtype, int M, int x_dtype, int K, int N, hipStream_t st) {
   const int R = x_dtype == MIQ_F32 ? 2 : 1, Mx = R * M;
   const Plan pl = plan(M, K, N, x_dtype);
@@ -704,7 +738,7 @@ static int workspace_call(const char* who, bool ok, int M, int K, int N, int x_d
 }
 
 template <bool NIB>
-static int stage(const void* x, int x_dtype, __half* xs, float* rs, float* rmax, int M, int K, hipStream_t st) {
+static int stage(const void* x, int x_dtype, __half* xs, uint2* rs, float* rmax, int M, int K, hipStream_t st) {
   if (x_dtype == MIQ_F32) {
     if ((size_t)K * 4 > 64 * 1024) {
       const int rc = require_lds("ggml_gemm staging", (size_t)K * 4);
@@ -737,7 +771,7 @@ static int gemm_call(const char* who, bool ok, const void* x, int x_dtype, const
   hipStream_t st = static_cast<hipStream_t>(stream);
   unsigned char* b = static_cast<unsigned char*>(workspace);
   __half* xs = reinterpret_cast<__half*>(b + L.xs);
-  float* rs = reinterpret_cast<float*>(b + L.rs);
+  uint2* rs = reinterpret_cast<uint2*>(b + L.rs);
   float* rmax = reinterpret_cast<float*>(b + L.rmax);
   float* part = reinterpret_cast<float*>(b + L.part);
   const int rc = is_nib(ggml_type) ? stage<true>(x, x_dtype, xs, rs, rmax, M, K, st)
