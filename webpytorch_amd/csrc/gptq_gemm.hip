@@ -141,9 +141,11 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(const __half* __restric
 
 // fp32 activations through the fp16 matrix cores: row m of x is scaled by 2^s (s making its
 // largest |x| just below 2^15) and split into hi = fp16(x 2^s) and lo = fp16(x 2^s - hi), staged
-// as rows m and M + m of a 2M-row problem (about 22 significant bits relative to the row's
-// largest value, no fp16 range limit; NaN or infinite rows keep scale 1 and propagate). The
-// GEMM's two result rows are added and scaled back by 2^-s (exact).
+// as rows 2m and 2m + 1 of a 2M-row problem (about 22 significant bits relative to the row's
+// largest value, no fp16 range limit; NaN or infinite rows keep scale 1 and propagate). A lane of
+// the GEMM holds both result rows (rows 4 kb + r of a 16-row tile), adds them and scales them back
+// by 2^-s (exact) as it stores. A pass of its own over both fp32 rows took 16 us of 156 at 1500
+// rows, 3584 -> 4608, and 4 x 4.9 us a layer of a 700-token prefill.
 __device__ __forceinline__ int f32_row_exp(float m) {
   if (!(m > 0.f) || !(m <= 3.4e38f)) return 0;
   int ex;
@@ -151,9 +153,9 @@ __device__ __forceinline__ int f32_row_exp(float m) {
   return min(max(15 - ex, -126), 126);  // any finite maximum lands below 2^15; 2^s stays finite
 }
 
-// Stage row m of fp32 x (gathered through perm if PERM) as hi (row m) and lo (row M + m) of the
+// Stage row m of fp32 x (gathered through perm if PERM) as hi (row 2m) and lo (row 2m + 1) of the
 // 2M-row stage-major pair-ordered layout, and record the row's largest |x| (NaN if it holds one)
-// in rmax[m] for the combine. The row goes through LDS (its maximum sets the scale before any
+// in rmax[m] for the GEMM's epilogue. The row goes through LDS (its maximum sets the scale before any
 // value is split). Grid (M), dynamic LDS 4 K bytes.
 template <int BITS, bool PERM>
 __global__ __launch_bounds__(256) void stage_rows_f32_kernel(const float* __restrict__ x, const int32_t* __restrict__ perm,
@@ -204,26 +206,11 @@ __global__ __launch_bounds__(256) void stage_rows_f32_kernel(const float* __rest
               ((uint32_t)__half_as_ushort(__float2half_rn(a1 - __half2float(h1))) << 16);
     }
     const int k = i * 8;
-    *reinterpret_cast<uint4*>(xp + ((size_t)(k / KC) * M2 + m) * KC + k % KC) =
+    *reinterpret_cast<uint4*>(xp + ((size_t)(k / KC) * M2 + 2 * m) * KC + k % KC) =
         pair_order8<BITS>(make_uint4(hi[0], hi[1], hi[2], hi[3]));
-    *reinterpret_cast<uint4*>(xp + ((size_t)(k / KC) * M2 + M + m) * KC + k % KC) =
+    *reinterpret_cast<uint4*>(xp + ((size_t)(k / KC) * M2 + 2 * m + 1) * KC + k % KC) =
         pair_order8<BITS>(make_uint4(lo[0], lo[1], lo[2], lo[3]));
   }
-}
-
-// out[m][n] = (y2[m][n] + y2[M + m][n]) 2^-s(m) + bias[n]. Grid (N/4/256 rounded up, M).
-template <typename OT>
-__global__ __launch_bounds__(256) void combine_rows_kernel(const float* __restrict__ y2, const float* __restrict__ rmax,
-                                                           const float* __restrict__ bias, OT* __restrict__ out, int M,
-                                                           int N) {
-  const int m = blockIdx.y, n = (blockIdx.x * 256 + threadIdx.x) * 4;
-  if (n >= N) return;
-  const float un = ldexpf(1.f, -f32_row_exp(rmax[m]));
-  const float4 a = *reinterpret_cast<const float4*>(y2 + (size_t)m * N + n);
-  const float4 b = *reinterpret_cast<const float4*>(y2 + (size_t)(M + m) * N + n);
-  const float r[4] = {(a.x + b.x) * un, (a.y + b.y) * un, (a.z + b.z) * un, (a.w + b.w) * un};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) out[(size_t)m * N + n + j] = from_f32<OT>(bias ? r[j] + bias[n + j] : r[j]);
 }
 
 // Launches the staging of x (gathered through perm if non-null) into xp with stage width KC.
@@ -278,8 +265,8 @@ template <int BITS, int TM, int CB, int KC, typename ST, typename OT>
 __global__ __attribute__((amdgpu_flat_work_group_size(1, TM * CB <= 4 ? 768 : 512),
                           amdgpu_waves_per_eu(TM * CB <= 4 ? 3 : 2, TM * CB <= 4 ? 3 : 2))) void gptq_gemm_kernel(
     const __half* __restrict__ xp, const uint32_t* __restrict__ qw, const uint32_t* __restrict__ qz,
-    const ST* __restrict__ sc, const float* __restrict__ bias, OT* __restrict__ out, float* __restrict__ ws,
-    int* __restrict__ counters, int M, int K, int N, int gs, float zoff, int stages_per_wg, int ksplit, int ntiles,
+    const ST* __restrict__ sc, const float* __restrict__ bias, const float* __restrict__ rmax,
+    OT* __restrict__ out, float* __restrict__ ws, int* __restrict__ counters, int M, int K, int N, int gs, float zoff, int stages_per_wg, int ksplit, int ntiles,
     int mtiles) {
   using G = GemmShape<BITS, TM, CB, KC, ST>;
   constexpr int PER = G::PER, STEPS = G::STEPS, RB = G::RB, NBUF = G::NBUF, NB2 = G::NB2, P2 = G::P2, NIW = G::NIW;
@@ -490,12 +477,29 @@ __global__ __attribute__((amdgpu_flat_work_group_size(1, TM * CB <= 4 ? 768 : 51
   }
   const bool producer = copier || half == 1;  // from here on, only the barriers
 
-  // ---- epilogue: D[row = m0 + 16 t + 4 kb + r][col = ncol + s] = acc[t][s][r] ----
-  if (ksplit == 1) {
-    if (producer || !colok) return;
+  // ---- epilogue: D[row = m0 + 16 t + 4 kb + r][col = ncol + s] = v[t][s][r]; with rmax, rows 2m
+  // and 2m + 1 are the planes of output row m (M is even) ----
+  auto store = [&](const float4v(&v)[TM][CB]) __attribute__((always_inline)) {
     float bv[CB];
 #pragma unroll
     for (int s = 0; s < CB; ++s) bv[s] = bias ? bias[ncol + s] : 0.f;
+    if (rmax) {
+#pragma unroll
+      for (int t = 0; t < TM; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+          const int row = m0 + 16 * t + 4 * kb + r;
+          if (row >= M) continue;
+          const float un = ldexpf(1.f, -f32_row_exp(rmax[row >> 1]));
+          OT* o = out + (size_t)(row >> 1) * N + ncol;
+#pragma unroll
+          for (int s = 0; s < CB; ++s) {
+            const float y = (v[t][s][r] + v[t][s][r + 1]) * un;
+            o[s] = from_f32<OT>(bias ? y + bv[s] : y);
+          }
+        }
+      return;
+    }
 #pragma unroll
     for (int t = 0; t < TM; ++t)
 #pragma unroll
@@ -504,8 +508,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(1, TM * CB <= 4 ? 768 : 51
         if (row >= M) continue;
         OT* o = out + (size_t)row * N + ncol;
 #pragma unroll
-        for (int s = 0; s < CB; ++s) o[s] = from_f32<OT>(acc[t][s][r] + bv[s]);
+        for (int s = 0; s < CB; ++s) o[s] = from_f32<OT>(v[t][s][r] + bv[s]);
       }
+  };
+  if (ksplit == 1) {
+    if (!producer && colok) store(acc);
     return;
   }
   // split K: device-scope stores of the slice, count in, the last workgroup sums the slices
@@ -574,18 +581,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(1, TM * CB <= 4 ? 768 : 51
             for (int r = 0; r < 4; ++r) sum[t][s][r] += own ? acc[t][s][r] : v[u][t][r][s];
       }
     }
-    if (colok) {
-#pragma unroll
-      for (int t = 0; t < TM; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = m0 + 16 * t + 4 * kb + r;
-          if (row >= M) continue;
-          OT* o = out + (size_t)row * N + ncol;
-#pragma unroll
-          for (int s = 0; s < CB; ++s) o[s] = from_f32<OT>(sum[t][s][r] + (bias ? bias[ncol + s] : 0.f));
-        }
-    }
+    if (colok) store(sum);
   }
   if (tid == 0) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-armed
 }
@@ -644,68 +640,68 @@ static int gemm_plan(int M, int K, int N, int gs, int bits, GemmPlan* p) {
 
 template <int BITS, int TM, int CB, int KC, typename ST, typename OT>
 static int launch_gemm(const GemmPlan& p, const __half* xp, const int32_t* qw, const int32_t* qz, const void* sc,
-                       const float* bias, void* out, void* ws, int M, int K, int N, int gs, float zoff, hipStream_t st) {
+                       const float* bias, const float* rmax, void* out, void* ws, int M, int K, int N, int gs, float zoff,
+                       hipStream_t st) {
   int* counters = static_cast<int*>(ws);
   float* partials = reinterpret_cast<float*>(static_cast<char*>(ws) + kCounterBytes);
   const int grid = p.ntiles * p.mtiles * p.ksplit;
   hipLaunchKernelGGL((gptq_gemm_kernel<BITS, TM, CB, KC, ST, OT>), dim3(grid), dim3(GemmShape<BITS, TM, CB, KC, ST>::THREADS), 0, st, xp,
                      reinterpret_cast<const uint32_t*>(qw), reinterpret_cast<const uint32_t*>(qz),
-                     static_cast<const ST*>(sc), bias, static_cast<OT*>(out), partials, counters, M, K, N, gs, zoff,
+                     static_cast<const ST*>(sc), bias, rmax, static_cast<OT*>(out), partials, counters, M, K, N, gs, zoff,
                      p.stages_per_wg, p.ksplit, p.ntiles, p.mtiles);
   return check_launch("gptq_gemm");
 }
 
 template <int BITS, int TM, int CB, int KC>
 static int gemm_types(const GemmPlan& p, const __half* xp, const int32_t* qw, const int32_t* qz, const void* sc,
-                      int sd, const float* bias, void* out, int od, void* ws, int M, int K, int N, int gs, float zoff,
+                      int sd, const float* bias, const float* rmax, void* out, int od, void* ws, int M, int K, int N, int gs, float zoff,
                       hipStream_t st) {
   if (sd == MIQ_F16) {
     if (od == MIQ_F16)
-      return launch_gemm<BITS, TM, CB, KC, __half, __half>(p, xp, qw, qz, sc, bias, out, ws, M, K, N, gs, zoff, st);
-    return launch_gemm<BITS, TM, CB, KC, __half, float>(p, xp, qw, qz, sc, bias, out, ws, M, K, N, gs, zoff, st);
+      return launch_gemm<BITS, TM, CB, KC, __half, __half>(p, xp, qw, qz, sc, bias, rmax, out, ws, M, K, N, gs, zoff, st);
+    return launch_gemm<BITS, TM, CB, KC, __half, float>(p, xp, qw, qz, sc, bias, rmax, out, ws, M, K, N, gs, zoff, st);
   }
   if (od == MIQ_F16)
-    return launch_gemm<BITS, TM, CB, KC, float, __half>(p, xp, qw, qz, sc, bias, out, ws, M, K, N, gs, zoff, st);
-  return launch_gemm<BITS, TM, CB, KC, float, float>(p, xp, qw, qz, sc, bias, out, ws, M, K, N, gs, zoff, st);
+    return launch_gemm<BITS, TM, CB, KC, float, __half>(p, xp, qw, qz, sc, bias, rmax, out, ws, M, K, N, gs, zoff, st);
+  return launch_gemm<BITS, TM, CB, KC, float, float>(p, xp, qw, qz, sc, bias, rmax, out, ws, M, K, N, gs, zoff, st);
 }
 
 template <int BITS, int KC>
 static int gemm_tiles(const GemmPlan& p, const __half* xp, const int32_t* qw, const int32_t* qz, const void* sc,
-                      int sd, const float* bias, void* out, int od, void* ws, int M, int K, int N, int gs, float zoff,
+                      int sd, const float* bias, const float* rmax, void* out, int od, void* ws, int M, int K, int N, int gs, float zoff,
                       hipStream_t st) {
-  if (p.tm == 4 && p.cb == 2) return gemm_types<BITS, 4, 2, KC>(p, xp, qw, qz, sc, sd, bias, out, od, ws, M, K, N, gs, zoff, st);
-  if (p.tm == 2 && p.cb == 2) return gemm_types<BITS, 2, 2, KC>(p, xp, qw, qz, sc, sd, bias, out, od, ws, M, K, N, gs, zoff, st);
-  if (p.tm == 1 && p.cb == 2) return gemm_types<BITS, 1, 2, KC>(p, xp, qw, qz, sc, sd, bias, out, od, ws, M, K, N, gs, zoff, st);
+  if (p.tm == 4 && p.cb == 2) return gemm_types<BITS, 4, 2, KC>(p, xp, qw, qz, sc, sd, bias, rmax, out, od, ws, M, K, N, gs, zoff, st);
+  if (p.tm == 2 && p.cb == 2) return gemm_types<BITS, 2, 2, KC>(p, xp, qw, qz, sc, sd, bias, rmax, out, od, ws, M, K, N, gs, zoff, st);
+  if (p.tm == 1 && p.cb == 2) return gemm_types<BITS, 1, 2, KC>(p, xp, qw, qz, sc, sd, bias, rmax, out, od, ws, M, K, N, gs, zoff, st);
   if constexpr (BITS == 4 || KC < 128) {  // int8 weights with 4 columns a lane take 64-wide stages
-    if (p.tm == 4 && p.cb == 4) return gemm_types<BITS, 4, 4, KC>(p, xp, qw, qz, sc, sd, bias, out, od, ws, M, K, N, gs, zoff, st);
-    if (p.tm == 2 && p.cb == 4) return gemm_types<BITS, 2, 4, KC>(p, xp, qw, qz, sc, sd, bias, out, od, ws, M, K, N, gs, zoff, st);
-    if (p.tm == 1 && p.cb == 4) return gemm_types<BITS, 1, 4, KC>(p, xp, qw, qz, sc, sd, bias, out, od, ws, M, K, N, gs, zoff, st);
+    if (p.tm == 4 && p.cb == 4) return gemm_types<BITS, 4, 4, KC>(p, xp, qw, qz, sc, sd, bias, rmax, out, od, ws, M, K, N, gs, zoff, st);
+    if (p.tm == 2 && p.cb == 4) return gemm_types<BITS, 2, 4, KC>(p, xp, qw, qz, sc, sd, bias, rmax, out, od, ws, M, K, N, gs, zoff, st);
+    if (p.tm == 1 && p.cb == 4) return gemm_types<BITS, 1, 4, KC>(p, xp, qw, qz, sc, sd, bias, rmax, out, od, ws, M, K, N, gs, zoff, st);
   }
   return ::miq::fail(MIQ_ERR_UNSUPPORTED, "gptq_gemm: no kernel for tile %dx%d, stage %d", p.tm, p.cb, KC);
 }
 
 template <int BITS>
 static int gemm_dispatch(const GemmPlan& p, const __half* xp, const int32_t* qw, const int32_t* qz, const void* sc,
-                         int sd, const float* bias, void* out, int od, void* ws, int M, int K, int N, int gs,
+                         int sd, const float* bias, const float* rmax, void* out, int od, void* ws, int M, int K, int N, int gs,
                          float zoff, hipStream_t st) {
-  if (p.kc == 128) return gemm_tiles<BITS, 128>(p, xp, qw, qz, sc, sd, bias, out, od, ws, M, K, N, gs, zoff, st);
-  if (p.kc == 64) return gemm_tiles<BITS, 64>(p, xp, qw, qz, sc, sd, bias, out, od, ws, M, K, N, gs, zoff, st);
-  return gemm_tiles<BITS, 32>(p, xp, qw, qz, sc, sd, bias, out, od, ws, M, K, N, gs, zoff, st);
+  if (p.kc == 128) return gemm_tiles<BITS, 128>(p, xp, qw, qz, sc, sd, bias, rmax, out, od, ws, M, K, N, gs, zoff, st);
+  if (p.kc == 64) return gemm_tiles<BITS, 64>(p, xp, qw, qz, sc, sd, bias, rmax, out, od, ws, M, K, N, gs, zoff, st);
+  return gemm_tiles<BITS, 32>(p, xp, qw, qz, sc, sd, bias, rmax, out, od, ws, M, K, N, gs, zoff, st);
 }
 
 int check_gptq_dims(const char* who, int K, int N, int gs, int bits);
 
 // Workspace layout of the fp32-activation GEMM: the 2M-row GEMM's own workspace (counters,
-// partials, staged rows), then its fp32 result [2M][N], then the row maxima [M].
+// partials, staged rows), then the row maxima [M].
 struct F32Plan {
   GemmPlan g;
-  size_t y2_off, rmax_off, ws_bytes;
+  size_t rmax_off, ws_bytes;
 };
 static int f32_plan(int M, int K, int N, int gs, int bits, F32Plan* p) {
   int rc = gemm_plan(2 * M, K, N, gs, bits, &p->g);
   if (rc) return rc;
-  p->y2_off = (p->g.ws_bytes + 255) & ~(size_t)255;
-  p->rmax_off = p->y2_off + (((size_t)2 * M * N * 4 + 255) & ~(size_t)255);
+  p->rmax_off = (p->g.ws_bytes + 255) & ~(size_t)255;
   p->ws_bytes = p->rmax_off + (((size_t)M * 4 + 255) & ~(size_t)255);
   return MIQ_OK;
 }
@@ -753,7 +749,6 @@ extern "C" int miq_gptq_gemm_f32x(const float* x, const int32_t* perm, const int
   hipStream_t st = static_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
   __half* xp = reinterpret_cast<__half*>(ws + kCounterBytes + p.g.partial_bytes);
-  float* y2 = reinterpret_cast<float*>(ws + p.y2_off);
   float* rmax = reinterpret_cast<float*>(ws + p.rmax_off);
   const size_t lds = (size_t)K * 4;
   if (lds > 64 * 1024 && (rc = require_lds("gptq_gemm_f32x staging", lds))) return rc;
@@ -767,17 +762,10 @@ extern "C" int miq_gptq_gemm_f32x(const float* x, const int32_t* perm, const int
 #undef MIQ_F32_STAGE
   rc = check_launch("gptq_gemm_f32x staging");
   if (rc) return rc;
-  rc = bits == 4 ? gemm_dispatch<4>(p.g, xp, qweight, qzeros, scales, scales_dtype, nullptr, y2, MIQ_F32, workspace,
-                                    2 * M, K, N, gs, zero_offset, st)
-                 : gemm_dispatch<8>(p.g, xp, qweight, qzeros, scales, scales_dtype, nullptr, y2, MIQ_F32, workspace,
-                                    2 * M, K, N, gs, zero_offset, st);
-  if (rc) return rc;
-  const dim3 g((N / 4 + 255) / 256, M);
-  if (out_dtype == MIQ_F16)
-    hipLaunchKernelGGL(combine_rows_kernel<__half>, g, dim3(256), 0, st, y2, rmax, bias, static_cast<__half*>(out), M, N);
-  else
-    hipLaunchKernelGGL(combine_rows_kernel<float>, g, dim3(256), 0, st, y2, rmax, bias, static_cast<float*>(out), M, N);
-  return check_launch("gptq_gemm_f32x combine");
+  return bits == 4 ? gemm_dispatch<4>(p.g, xp, qweight, qzeros, scales, scales_dtype, bias, rmax, out, out_dtype,
+                                      workspace, 2 * M, K, N, gs, zero_offset, st)
+                   : gemm_dispatch<8>(p.g, xp, qweight, qzeros, scales, scales_dtype, bias, rmax, out, out_dtype,
+                                      workspace, 2 * M, K, N, gs, zero_offset, st);
 }
 
 extern "C" int miq_gptq_gemm_workspace(int M, int K, int N, int gs, int bits, size_t* bytes) {
@@ -840,8 +828,8 @@ extern "C" int miq_gptq_gemm(const void* x, const int32_t* perm, const int32_t* 
   rc = bits == 4 ? stage_rows<4>(xin, perm, xp, M, K, p.kc, st) : stage_rows<8>(xin, perm, xp, M, K, p.kc, st);
   if (rc) return rc;
   if (bits == 4)
-    return gemm_dispatch<4>(p, xp, qweight, qzeros, scales, scales_dtype, bias, out, out_dtype, workspace, M, K, N, gs,
-                            zero_offset, st);
-  return gemm_dispatch<8>(p, xp, qweight, qzeros, scales, scales_dtype, bias, out, out_dtype, workspace, M, K, N, gs,
-                          zero_offset, st);
+    return gemm_dispatch<4>(p, xp, qweight, qzeros, scales, scales_dtype, bias, nullptr, out, out_dtype, workspace, M, K,
+                            N, gs, zero_offset, st);
+  return gemm_dispatch<8>(p, xp, qweight, qzeros, scales, scales_dtype, bias, nullptr, out, out_dtype, workspace, M, K, N,
+                          gs, zero_offset, st);
 }
