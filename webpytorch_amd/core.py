@@ -20,6 +20,8 @@ from ._lib import MIQ_F16, MIQ_F32
 
 # M above which a GPTQ matmul leaves the GEMV kernel for the MFMA GEMM.
 GEMV_MAX_M = 8
+# Products from which 2 to GEMV_MAX_M fp16 rows may leave it too (`_few_rows_gemm_taken`).
+FEW_ROWS_MIN = 1 << 25
 
 
 # ---- plumbing --------------------------------------------------------------------------
@@ -211,6 +213,26 @@ def _gptq_path(M, xdt):
 
 
 # ---- GPTQ ----------------------------------------------------------------------------
+def _few_rows_gemm_taken(xf, qweight, scales, K, N, gs, bits, zoff, perm, ws):
+    """Whether 2 to GEMV_MAX_M fp16 rows run on the few-row matrix-core kernel behind
+    `miq_gptq_gemm` rather than the GEMV, whose vector work grows with the rows. The shapes are
+    those that kernel covers (int4, groups of 128, rows in k order; at most 7680 outputs where it
+    splits K, which it does not for 8129 outputs and more with K to 4096). Both cost the host 18 us
+    a call; the GEMV's kernel passes that from about 2^25 products on (us a call, few-row / GEMV:
+    4096 -> 4096 18 / 26 at 8 rows, 18 / 18 at 6; 4096 -> 11008 18 / 20 at 6; 11008 -> 4096 18 / 23
+    at 2, 18 / 50 at 8). A workspace handed in, or held while a graph is captured, has to suffice."""
+    M = int(xf.shape[0])
+    if not (1 < M <= GEMV_MAX_M and M * K * N >= FEW_ROWS_MIN and bits == 4 and gs == 128 and perm is None
+            and xf.dtype == torch.float16 and float(zoff).is_integer() and 0 <= zoff <= 8 and K % 128 == 0
+            and K <= 16384 and N % 8 == 0 and (N <= 7680 or (N > 8128 and K <= 4096))
+            and qweight.data_ptr() % 16 == 0 and scales.data_ptr() % 16 == 0):
+        return False
+    need = gemm_workspace_bytes(M, K, N, gs, bits)
+    if ws is not None:
+        return ws.numel() >= need and ws.data_ptr() % 256 == 0
+    return not torch.cuda.is_current_stream_capturing() or workspace_holds(need)
+
+
 def gptq_dequant(qweight, qzeros, scales, K, N, gs, bits, zoff=0.0, g_idx=None):
     """Full fp32 weight (K, N); bit-exact with the reference's dequant for integer zoff."""
     out = torch.empty((K, N), dtype=torch.float32, device=device())
@@ -222,21 +244,24 @@ def gptq_dequant(qweight, qzeros, scales, K, N, gs, bits, zoff=0.0, g_idx=None):
 def _gptq_matmul(xf, qweight, qzeros, scales, K, N, gs, bits, zoff=0.0, *, bias=None, perm=None,
                  out_dtype=None, out=None, ws=None, _check=True):
     """xf (M, K) @ dequant(W) (+ bias) -> (M, N) on the current stream
-    (`webtorch/_core.py:4008-4043`). Up to GEMV_MAX_M rows run the split-K GEMV; more rows
+    (`webtorch/_core.py:4008-4043`). Up to GEMV_MAX_M rows run the split-K GEMV (or, where
+    `_few_rows_gemm_taken` says so, the few-row matrix-core kernel); more rows
     run the matrix-core GEMM (fp32 activations as row-scaled fp16 hi/lo pairs of rows). The
     first call of each kernel class on a device runs its known-answer check (RuntimeError if
     it fails)."""
     M = int(xf.shape[0])
-    if _check:
-        selfcheck_gptq(M, xf.dtype, bits, gs, scales.dtype, zoff)
+    xf = aligned16(xf)
+    few = (1 < M <= GEMV_MAX_M and M * K * N >= FEW_ROWS_MIN
+           and _few_rows_gemm_taken(xf, qweight, scales, K, N, gs, bits, zoff, perm, ws))
+    if _check:  # 12 rows are the few-row kernel's class
+        selfcheck_gptq(12 if few else M, xf.dtype, bits, gs, scales.dtype, zoff)
     od = out_dtype or torch.float32
     if out is None:
         out = torch.empty((M, N), dtype=od, device=xf.device)
     if M == 0:
         return out
-    xf = aligned16(xf)
     xd = dtype_code(xf)
-    if M > GEMV_MAX_M and xd == MIQ_F16 and float(zoff).is_integer() and 0 <= zoff <= 8:
+    if few or M > GEMV_MAX_M and xd == MIQ_F16 and float(zoff).is_integer() and 0 <= zoff <= 8:
         if ws is None:
             ws = workspace(gemm_workspace_bytes(M, K, N, gs, bits))
         _lib.call("miq_gptq_gemm", ptr(xf), ptr(perm), ptr(qweight), ptr(qzeros), ptr(scales),
@@ -551,7 +576,7 @@ def ggml_matmul(xf, packed, type_name, K, N, bias=None, out_dtype=torch.float32,
                                                                            int(N) * rowb))
     xf = aligned16(as_activation(xf).contiguous())
     M = int(xf.shape[0])
-    nibble = _nibble_gemm_taken(type_name, M, int(K), int(N), dtype_code(xf), packed)
+    nibble = M > GGML_GEMV_MAX_M and _nibble_gemm_taken(type_name, M, int(K), int(N), dtype_code(xf), packed)
     gemm = nibble or _ggml_gemm_taken(type_name, M, int(K))
     mode = -1 if gemm else (M if M <= 2 else 0)
     if _check and M and _first_use(("ggml", type_name, mode)):
