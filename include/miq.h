@@ -67,9 +67,10 @@ int miq_gptq_repack_rows(const int32_t* qweight, const int32_t* perm, int32_t* o
  * escape masks, shared by every split-K entry point, that must be zero before the first call
  * on it; every call leaves them zero again. Partial sums, escape slots and staged activations
  * follow them. One workspace must not serve two calls that run concurrently.
- * Split-K sums are exact for every input: a K-slice partial that is NaN, infinite or of
- * magnitude >= 2^22 (beyond the fixed-point words) reaches the final sum as an fp32 value, so
- * NaN and infinities propagate as in an fp32 sum. (The one-row int4 kernel holds each 64-k step
+ * The one-row int4 kernel sums its K-slices in fixed point on a grid of 2^-24, so outputs much
+ * below 1 keep fewer digits (about 2^-24 per slice, whatever the output's size); a partial that is
+ * NaN, infinite or of magnitude >= 2^22 (beyond the words) reaches the final sum as an fp32 value,
+ * so NaN and infinities propagate as in an fp32 sum. The other products sum fp32 partials. (The one-row int4 kernel holds each 64-k step
  * of x in fixed point at the step's own scale, which a non-finite value has not: such a step
  * scales its products by NaN, so an infinite x gives NaN, not +-Inf, in the outputs it
  * reaches.) */
@@ -137,7 +138,7 @@ int miq_gptq_gemm_workspace(int M, int K, int N, int gs, int bits, size_t* bytes
  * scales fp16|fp32, out fp16|fp32. Requires x and qweight 16-byte aligned, N % 4 == 0 and
  * gs in {32, 64} or a multiple of 128. workspace as for miq_gptq_gemv. Up to 16 rows of int4
  * with gs 128 run a kernel that streams the weights like the GEMV (all loads issued up front,
- * K split over waves and workgroups, deterministic fixed-point slice sums); more rows run the
+ * K split over waves and workgroups, fp32 slice sums added in slice order); more rows run the
  * tiled LDS-pipelined kernel.
  * Replaces: `_gptq_matmul` M > 1 dispatch to the tiled `_GPTQ_WGSL` kernel
  * (webtorch/_core.py:3833-3888, 3995-4027) and the bias add of `QuantizedLinear.forward`

@@ -94,7 +94,7 @@ def test_gemm_repeated_calls_are_deterministic(gpu):
 ])
 def test_few_row_gemm(gpu, K, N, M, sdt, zoff, bias, act):
     """The few-row matrix-core product (M <= 16, gs = 128): exact bf16 halves of the fp16 rows,
-    per-group folds, a fixed-point split-K; called through miq_gptq_gemm."""
+    per-group folds, fp32 split-K sums; called through miq_gptq_gemm."""
     import torch
     from webpytorch_amd import core
     L = synth.gptq_layer(60 + M, K, N, 128, 4, act_order=act)
@@ -117,7 +117,7 @@ def test_few_row_gemm(gpu, K, N, M, sdt, zoff, bias, act):
     if b is not None:
         ref = ref + b
     _check(got, ref, rel=1e-5)
-    for _ in range(2):  # the fixed-point words re-zero: repeated calls agree bit for bit
+    for _ in range(2):  # the arrival counters re-zero: repeated calls agree bit for bit
         core._lib.call("miq_gptq_gemm", core.ptr(xd), core.ptr(ql.perm), core.ptr(ql.qweight),
                        core.ptr(ql.qzeros), core.ptr(ql.scales), core.dtype_code(ql.scales), core.ptr(ql.bias),
                        core.ptr(out), core.dtype_code(out), M, K, N, 128, 4, float(zoff), core.ptr(ws), ws.numel(),

@@ -2,14 +2,14 @@
 
 The reference multiplies in numpy fp32 (`_gptq_matmul_np`, `webtorch/_core.py:4046-4072`), so a
 NaN activation makes every output NaN, an infinite one makes each output +-Inf (or NaN where the
-weight is zero), and large finite activations give large finite outputs. The split-K kernels
-here meet their K-slices in fixed-point words; partials those cannot hold take an exact fp32
-escape, so the same inputs must give the same non-finite pattern and, for large finite values,
+weight is zero), and large finite activations give large finite outputs. The one-row kernel
+meets its K-slices in fixed-point words; partials those cannot hold take an exact fp32
+escape; the others sum fp32 partials. So the same inputs must give the same non-finite pattern and, for large finite values,
 the same numbers to fp32 accuracy.
 
 Paths: one row of fp32 x (matrix-core GEMV, fixed-point split-K), four rows of fp32 x (the
-VALU GEMV), four rows of fp16 x (few-row matrix-core GEMM, fixed-point split-K) and 64 rows of
-fp16 x (tiled MFMA GEMM, fp32 split-K partials).
+VALU GEMV), four rows of fp16 x (the VALU GEMV at this size; the few-row matrix-core kernel's turn is
+in test_gpu_few_rows.py) and 64 rows of fp16 x (tiled MFMA GEMM, fp32 split-K partials).
 """
 import numpy as np
 import pytest

@@ -20,9 +20,15 @@
 // Activations are staged in LDS in the pair order of the B halves (k 0, 4, 1, 5, 2, 6, 3, 7).
 //
 // Reduction. The 4 waves' sums meet in LDS (wave order, deterministic), each wave then finishing
-// a quarter of the outputs. With one K-slice it writes y; with several, each output's slices
-// meet in a fixed-point word of the workspace's zeroed counter region (mma_tile.h: fix_add),
-// whose last arrival writes y.
+// a quarter of the outputs. With one K-slice it writes y; with several, each workgroup leaves its
+// fp32 sums in the workspace and counts itself in at the tile's counter (the workspace's zeroed
+// counter region; every wave by itself, as its outputs are its own), and the last adds the slices
+// in slice order and writes y. Sums in 64-bit words on a fixed grid of 2^-24, which took one round
+// trip less, stood 4e-5 from float64 for outputs near 1e-3 and 4e-4 near 1e-4; these stand 0.7 to
+// 1.2e-7 at every magnitude, and each counter has a 128-byte line of its own: counters side by side
+// queue in their line (16384 -> 1024, 32 slices of 16 tiles: 16.4 us, 8.0 apart). Kernel time, us,
+// fixed grid / fp32 sums: 4096 -> 4096 6.1 / 6.6 at 2 rows, 7.3 / 6.9 at 8, 9.2 / 8.2 at 16;
+// 11008 -> 4096 9.3 / 10.1, 10.6 / 10.4, 12.4 / 12.3; 4864 -> 896 4.4 / 5.0, 5.7 / 5.3, 6.8 / 6.2.
 //
 // x is read as fp16 rows (row-major), or, for act-order weights (rows stored by group), from the
 // copy the prefill GEMM's gather pass makes (pair order, stage-major with 128-wide stages).
@@ -37,6 +43,9 @@ namespace gs {
 using namespace mt;
 
 constexpr int kGsTargetWgs = 512;     // split K until the grid has this many workgroups
+constexpr int kGsMaxSlices = 32, kGsMaxTiles = 256;  // of a split product
+constexpr int kCtrStride = 32;                       // ints between counters: a 128-byte line each
+static_assert(kGsMaxTiles * 4 * kCtrStride * sizeof(int) <= kCounterBytes, "counters fit their region");
 constexpr int kGsWideMinTiles = 128;  // from this many column tiles, 16 waves cover all of K
 
 constexpr int kXkc = 128;  // stage width of the gathered copy
@@ -54,9 +63,8 @@ __global__ __launch_bounds__(NWV * 64) void gemm_small_kernel(const __half* __re
                                                               const uint32_t* __restrict__ qz,
                                                               const ST* __restrict__ sc,
                                                               const float* __restrict__ bias, OT* __restrict__ out,
-                                                              unsigned long long* __restrict__ fixacc,
-                                                              float* __restrict__ side, int M, int K, int N,
-                                                              float zoff) {
+                                                              int* __restrict__ counters, float* __restrict__ side,
+                                                              int M, int K, int N, float zoff) {
   using SV = typename Scales4<ST>::T;
   constexpr int NT = NWV * 64;         // threads
   constexpr int NG = SPQ / 4;          // groups per wave
@@ -153,8 +161,7 @@ __global__ __launch_bounds__(NWV * 64) void gemm_small_kernel(const __half* __re
 #pragma unroll
     for (int r = 0; r < 4; ++r) red[(wave * NV + t * 4 + r) * 64 + lane] = acc[t][r];
   __syncthreads();
-  // each wave finishes NV / NWV of the lane's outputs (returning atomics of one wave complete
-  // one after another, so they are spread over the waves)
+  // each wave finishes NV / NWV of the lane's outputs
   constexpr int NW = NV / NWV;
   float ys[NW];
 #pragma unroll
@@ -176,25 +183,53 @@ __global__ __launch_bounds__(NWV * 64) void gemm_small_kernel(const __half* __re
     }
     return;
   }
-  // every atomic first, then the checks: the round trips overlap. The words of a tile are laid
-  // out [v][lane], so one atomic instruction covers 512 contiguous bytes.
-  const size_t w0 = (size_t)tile * NV * 64 + lane, nwords = (size_t)gridDim.x * NV * 64;
-  unsigned long long add[NW], old[NW];
+  // This slice's sums to its fp32 slots [slice][tile][thread][4] (a wave covers 1 KB; rows past M
+  // and columns past N are neither stored nor read), with device-scope stores, which reach the
+  // coherence point without a write-back of the XCD's L2. A wave's outputs are its own, so it waits
+  // for its stores and counts itself in alone, with no barrier; the last of the slices' waves reads
+  // every slice with device-scope loads after it has seen the final count, and adds them in slice
+  // order.
+  if constexpr (NW == 4) {  // only these split K
+    const bool live = 4 * (lane >> 4) < M && c + wave < N;  // v = 4 wave + r: rows 4 (lane >> 4) + r, column c + wave
+    const size_t stride = (size_t)gridDim.x * NT * NW;
+    float* slot = side + ((size_t)tile * NT + threadIdx.x) * NW;
+    if (live) {
+      uint64_t* d = reinterpret_cast<uint64_t*>(slot + sl * stride);
 #pragma unroll
-  for (int u = 0; u < NW; ++u) {
-    const int v = wave * NW + u, m = row_of(v), n = col_of(v);
-    add[u] = fix_word(ys[u]);
-    old[u] = 0;
-    if (m < M && n < N)
-      old[u] = fix_issue(fixacc + w0 + v * 64, add[u], ys[u], fix_esc(fixacc, w0 + v * 64, side, nwords), sl);
-  }
+      for (int u = 0; u < NW; u += 2)
+        __hip_atomic_store(d + u / 2,
+                           (uint64_t)__float_as_uint(ys[u]) | ((uint64_t)__float_as_uint(ys[u + 1]) << 32),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    int* ctr = counters + (tile * NWV + wave) * kCtrStride;
+    int seen = 0;
+    if (lane == 0) seen = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (uniform(seen) != kslices - 1) return;
+    if (lane == 0) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-armed
+    if (!live) return;
+    constexpr int KU = 16;  // slices whose loads are in flight at once
+    float y[NW] = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < kslices; k0 += KU) {
+      uint64_t p[KU][2];
 #pragma unroll
-  for (int u = 0; u < NW; ++u) {
-    const int v = wave * NW + u, m = row_of(v), n = col_of(v);
-    float r;
-    if (m < M && n < N &&
-        fix_finish(fixacc + w0 + v * 64, old[u], add[u], kslices, fix_esc(fixacc, w0 + v * 64, side, nwords), &r))
-      out[(size_t)m * N + n] = from_f32<OT>(bias ? r + bias[n] : r);
+      for (int i = 0; i < KU; ++i) {
+        const uint64_t* q = reinterpret_cast<const uint64_t*>(slot + min(k0 + i, kslices - 1) * stride);
+        p[i][0] = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        p[i][1] = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+#pragma unroll
+      for (int i = 0; i < KU; ++i)
+        if (k0 + i < kslices) {
+#pragma unroll
+          for (int u = 0; u < NW; ++u) y[u] += __uint_as_float((uint32_t)(p[i][u / 2] >> (32 * (u & 1))));
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < NW; ++u) {
+      const int v = wave * NW + u, m = row_of(v), n = col_of(v);
+      if (m < M) out[(size_t)m * N + n] = from_f32<OT>(bias ? y[u] + bias[n] : y[u]);
+    }
   }
 }
 
@@ -204,8 +239,8 @@ struct Plan {
 
 // Either 16 waves per workgroup covering all of K (no split: K <= 16 x 8 steps, and enough
 // 64-column tiles to occupy the chip), or 4 waves per workgroup with SPQ (steps per wave) the
-// largest whose grid still has ~a workgroup per CU. K-slices beyond one need a fixed-point word
-// per output ([tile][16][64] words).
+// largest whose grid still has ~a workgroup per CU. Split products stop at kGsMaxSlices slices and
+// kGsMaxTiles tiles, the largest this kernel was compared with the tiled GEMM at.
 static bool plan(int M, int K, int N, Plan* p) {
   if (M < 1 || M > 16 || K % 128 || N % 8) return false;
   const int steps = K / 32;
@@ -227,21 +262,19 @@ static bool plan(int M, int K, int N, Plan* p) {
     }
   }
   p->kslices = (steps + 4 * p->spq - 1) / (4 * p->spq);
-  if (p->kslices > kFixMaxSlices) return false;
-  if (p->kslices > 1 && (size_t)p->tiles * 16 * 64 > kFixMaxWords) return false;
-  return true;
+  return p->kslices == 1 || (p->kslices <= kGsMaxSlices && p->tiles <= kGsMaxTiles);
 }
 
 template <int NWV, int SPQ, bool XP>
 static void launch3(const Plan& pl, const __half* x, const int32_t* qw, const int32_t* qz, const void* sc, int sd,
-                    const float* bias, void* out, int od, unsigned long long* fixacc, float* side, int M, int K, int N,
-                    float zoff, hipStream_t st) {
+                    const float* bias, void* out, int od, int* counters, float* side, int M, int K, int N, float zoff,
+                    hipStream_t st) {
   const dim3 grid(pl.tiles, pl.kslices);
   const uint32_t* w = reinterpret_cast<const uint32_t*>(qw);
   const uint32_t* z = reinterpret_cast<const uint32_t*>(qz);
 #define MIQ_GS_LAUNCH(ST, OT)                                                                                      \
   hipLaunchKernelGGL((gemm_small_kernel<NWV, SPQ, XP, ST, OT>), grid, dim3(NWV * 64), 0, st, x, w, z,            \
-                     static_cast<const ST*>(sc), bias, static_cast<OT*>(out), fixacc, side, M, K, N, zoff)
+                     static_cast<const ST*>(sc), bias, static_cast<OT*>(out), counters, side, M, K, N, zoff)
   if (sd == MIQ_F16) {
     if (od == MIQ_F16) MIQ_GS_LAUNCH(__half, __half);
     else MIQ_GS_LAUNCH(__half, float);
@@ -258,14 +291,14 @@ static void launch3(const Plan& pl, const __half* x, const int32_t* qw, const in
 static size_t xg_bytes(int M, int K) { return ((size_t)M * K * 2 + 255) & ~(size_t)255; }
 
 // Bytes of workspace gemm_small needs (0: none; SIZE_MAX: the shape is not covered): the counter
-// region, with perm the gathered copy of x, and with several K-slices the escape slots of the
-// fixed-point words ([kslices][words] floats).
+// region, with perm the gathered copy of x, and with several K-slices their fp32 sums
+// ([kslices][tiles][16 x 64]).
 size_t gemm_small_workspace(int M, int K, int N, int gs_, int bits, bool perm) {
   gs::Plan pl;
   if (bits != 4 || gs_ != 128 || !gs::plan(M, K, N, &pl)) return SIZE_MAX;
-  const size_t esc = pl.kslices > 1 ? (size_t)pl.kslices * pl.tiles * 16 * 64 * 4 : 0;
-  if (!perm) return pl.kslices > 1 ? kCounterBytes + esc : 0;
-  return kCounterBytes + xg_bytes(M, K) + esc;
+  const size_t part = pl.kslices > 1 ? (size_t)pl.kslices * pl.tiles * 16 * 64 * 4 : 0;
+  if (!perm) return pl.kslices > 1 ? kCounterBytes + part : 0;
+  return kCounterBytes + xg_bytes(M, K) + part;
 }
 
 // Launches the few-row product when it covers the shape; MIQ_ERR_UNSUPPORTED (before launching
@@ -279,15 +312,15 @@ int gemm_small(const __half* x, const __half* xg, const int32_t* qw, const int32
     return MIQ_ERR_UNSUPPORTED;
   if (pl.kslices > 1 && (!ws || ws_bytes < gemm_small_workspace(M, K, N, gs_, bits, xg != nullptr)))
     return MIQ_ERR_UNSUPPORTED;
-  unsigned long long* fixacc = pl.kslices > 1 ? static_cast<unsigned long long*>(ws) : nullptr;
+  int* counters = pl.kslices > 1 ? static_cast<int*>(ws) : nullptr;
   float* side = pl.kslices > 1 ? reinterpret_cast<float*>(static_cast<char*>(ws) + kCounterBytes +
                                                           (xg ? xg_bytes(M, K) : 0))
                                : nullptr;
   const __half* src = xg ? xg : x;
 #define MIQ_GS_CASE(NWV, SPQ)                                                                                      \
   if (pl.nwv == NWV && pl.spq == SPQ) {                                                                            \
-    if (xg) gs::launch3<NWV, SPQ, true>(pl, src, qw, qz, sc, sd, bias, out, od, fixacc, side, M, K, N, zoff, st); \
-    else gs::launch3<NWV, SPQ, false>(pl, src, qw, qz, sc, sd, bias, out, od, fixacc, side, M, K, N, zoff, st);   \
+    if (xg) gs::launch3<NWV, SPQ, true>(pl, src, qw, qz, sc, sd, bias, out, od, counters, side, M, K, N, zoff, st); \
+    else gs::launch3<NWV, SPQ, false>(pl, src, qw, qz, sc, sd, bias, out, od, counters, side, M, K, N, zoff, st);   \
     return check_launch("gemm_small");                                                                             \
   }
   MIQ_GS_CASE(4, 16) MIQ_GS_CASE(4, 8) MIQ_GS_CASE(4, 4) MIQ_GS_CASE(16, 8) MIQ_GS_CASE(16, 4)
