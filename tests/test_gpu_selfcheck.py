@@ -63,6 +63,33 @@ def test_check_raises_on_a_mismatch(gpu, monkeypatch):
         ql(torch.from_numpy(synth.activations(3, 1, 256, np.float32)))
 
 
+@pytest.mark.parametrize("type_name", ["Q4_K", "Q5_K", "Q6_K", "Q8_0", "Q4_0", "Q5_0", "IQ4_NL"])
+def test_gemm_check_runs_the_gemm(gpu, monkeypatch, type_name):
+    """The check of a prefill product launches the kernel it answers for, once, and raises for it."""
+    import torch
+    core = _fresh(monkeypatch)
+    entry = "miq_ggml_nibble_gemm" if type_name in ("Q4_0", "Q5_0", "IQ4_NL") else "miq_ggml_gemm"
+    launched, real = [], core._lib.call
+
+    def call(name, *args):
+        if not name.endswith("_workspace"):
+            launched.append(name)
+        return real(name, *args)
+    monkeypatch.setattr(core._lib, "call", call)
+    M, K, N = 512, 1024, 512  # 2^28 products: the nibble types' GEMM too
+    lin = core.GGMLLinear(synth.ggml_layer(type_name, 1, K, N), type_name, K, N)
+    x = torch.from_numpy(synth.activations(1, M, K, np.float32)).cuda()
+    for gemms in (2, 1):  # the check's launch and the product's, then the product's
+        launched.clear()
+        lin(x)
+        assert [n for n in launched if "gemm" in n or "gemv" in n] == [entry] * gemms
+    core._CHECKED.clear()
+    good = core._reference_product
+    monkeypatch.setattr(core, "_reference_product", lambda x, W: good(x, W) * 1.01)
+    with pytest.raises(RuntimeError, match="gemm kernel for %s.*wrong" % type_name):
+        lin(x)
+
+
 def test_no_check_under_graph_capture(gpu, monkeypatch):
     import torch
     core = _fresh(monkeypatch)

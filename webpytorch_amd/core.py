@@ -532,10 +532,21 @@ def _nibble_gemm_taken(type_name, M, K, N, x_dtype, packed):
             or workspace_holds(ggml_gemm_workspace_bytes(M, K, N, x_dtype, type_name)))
 
 
+def _ggml_gemm(xf, packed, type_name, K, N, bias, out):
+    """The type's matrix-core GEMM of rows xf (M, K) into out (M, N)."""
+    M, xd = int(xf.shape[0]), dtype_code(xf)
+    ws = workspace(ggml_gemm_workspace_bytes(M, K, N, xd, type_name))
+    _lib.call("miq_ggml_nibble_gemm" if type_name in GGML_NIBBLE_TYPES else "miq_ggml_gemm", ptr(xf), xd, ptr(packed),
+              _NATIVE_TYPES[type_name][2], ptr(bias), ptr(out), dtype_code(out), M, K, N, ptr(ws), ws.numel(),
+              stream_handle())
+
+
 def _ggml_selfcheck(type_name, mode):
     """Multiply two random blocks of `type_name` with the kernel of `mode` (rows 1, 2, 0 for 3
-    to GGML_GEMV_MAX_M, -1 for the matrix-core GEMM) and compare against the device's exact dequant of the same bytes times x in
-    float64; RuntimeError on a mismatch (`_ggml_selfcheck`, `webtorch/_core.py:3684-3717`).
+    to GGML_GEMV_MAX_M, -1 for the type's matrix-core GEMM, called by itself as the dispatch gives
+    the nibble types' only large products) and compare against the device's exact dequant of the
+    same bytes times x in float64; RuntimeError on a mismatch (`_ggml_selfcheck`,
+    `webtorch/_core.py:3684-3717`).
     Code and sub-scale bytes are uniform random (every byte pattern is a legal block); the fp16
     scale fields are drawn small and finite, where the reference redraws until they are."""
     from . import synth
@@ -548,7 +559,11 @@ def _ggml_selfcheck(type_name, mode):
     g = np.random.default_rng(vals)
     M = {0: 3, -1: 2 * GGML_GEMV_MAX_M + 1}.get(mode, mode)
     x = torch.from_numpy(g.standard_normal((M, K)).astype(np.float32)).to(device())
-    got = ggml_matmul(x, raw, type_name, K, 2, _check=False)
+    if mode < 0:
+        got = torch.empty((M, 2), dtype=torch.float32, device=x.device)
+        _ggml_gemm(x, raw, type_name, K, 2, None, got)
+    else:
+        got = ggml_matmul(x, raw, type_name, K, 2, _check=False)
     _check_close("the native ggml %s kernel for %s" % ("gemm" if mode < 0 else "gemv", type_name), got,
                  _reference_product(x, W.t()))
 
@@ -576,19 +591,15 @@ def ggml_matmul(xf, packed, type_name, K, N, bias=None, out_dtype=torch.float32,
                                                                            int(N) * rowb))
     xf = aligned16(as_activation(xf).contiguous())
     M = int(xf.shape[0])
-    nibble = M > GGML_GEMV_MAX_M and _nibble_gemm_taken(type_name, M, int(K), int(N), dtype_code(xf), packed)
-    gemm = nibble or _ggml_gemm_taken(type_name, M, int(K))
+    gemm = M > GGML_GEMV_MAX_M and (_nibble_gemm_taken(type_name, M, int(K), int(N), dtype_code(xf), packed)
+                                    or _ggml_gemm_taken(type_name, M, int(K)))
     mode = -1 if gemm else (M if M <= 2 else 0)
     if _check and M and _first_use(("ggml", type_name, mode)):
         _ggml_selfcheck(type_name, mode)
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype, device=xf.device)
     if gemm:  # prefill rows on the matrix cores
-        need = ggml_gemm_workspace_bytes(M, int(K), int(N), dtype_code(xf), type_name)
-        ws = workspace(need)
-        _lib.call("miq_ggml_nibble_gemm" if nibble else "miq_ggml_gemm", ptr(xf), dtype_code(xf), ptr(packed),
-                  _NATIVE_TYPES[type_name][2], ptr(bias), ptr(out), dtype_code(out), M, int(K), int(N), ptr(ws),
-                  ws.numel(), stream_handle())
+        _ggml_gemm(xf, packed, type_name, int(K), int(N), bias, out)
     elif type_name == "Q4_K":
         _lib.call("miq_q4k_gemv", ptr(xf), dtype_code(xf), ptr(packed), ptr(bias), ptr(out), dtype_code(out),
                   M, int(K), int(N), stream_handle())
