@@ -68,3 +68,19 @@ def test_non_finite_values_reach_only_their_queries(gpu, HD, bad):
     other = torch.arange(HD) != 5
     np.testing.assert_allclose(got[20:][..., other].numpy(), clean[20:][..., other].numpy(), rtol=0, atol=1e-5)
     assert not torch.isfinite(got[20:, :, 5]).any()
+
+
+@pytest.mark.parametrize("NH,NKV,HD", [(2, 1, 64), (2, 1, 128), (2, 1, 32)])
+@pytest.mark.parametrize("big", [1e36, 2e38])
+def test_values_near_the_fp32_range(gpu, NH, NKV, HD, big):
+    """Values whose sum over the keys is past the fp32 range: every output is a weighted mean of
+    them, so it is finite and, relatively, as near float64 as any other."""
+    import torch
+    g = torch.Generator().manual_seed(HD)
+    T, LMAX = 300, 1024
+    q, k = torch.randn((T, NH, HD), generator=g) * 0.1, torch.randn((NKV, LMAX, HD), generator=g)
+    v = (torch.rand((NKV, LMAX, HD), generator=g) * 0.5 + 0.5) * big
+    for pos in (0, LMAX - T):
+        got = run(q.cuda(), k.cuda(), v.cuda(), pos).cpu().double()
+        ref = want(q, k, v, pos)
+        assert float((got - ref).norm() / ref.norm()) < 2e-6

@@ -28,12 +28,17 @@ namespace miq {
 // Their probabilities are then 0, but 0 times a NaN or infinite value is NaN, so a masked block
 // whose values are not all finite is added key by key on the VALU instead, masked keys skipped.
 //
+// Sums of p v are divided by sum p at the end, so up to LMAX values add up undivided: p is held
+// times 2^-14 (exact, and gone with the division), which keeps them within the largest |v|.
+//
 // Bound: the fp32 matrix cores at long prompts, the round trips to the cache rows (the first
 // block's issued before the position is known) at short ones. Against one wave per (head,
 // token) with a score row in LDS, from position 0: 14 heads of 64, T = 64 6.1 -> 4.7 us, T = 700 138 -> 22,
 // T = 2000 997 -> 92; 28 heads of 128, T = 700 499 -> 58, T = 2000 4264 -> 339 (88 TFLOP/s); one
 // row behind 700 positions 37 -> 13 and 71 -> 19.
 constexpr int kAttWaves = 4;  // eight were slower from T = 700 on (T = 2000: 92 -> 106 us) and no faster below
+constexpr int kAttMaxKeys = 16384;           // LMAX
+constexpr float kAttUnit = 1.f / kAttMaxKeys;  // a probability of 1
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 // the maximum over the four lanes c, c + 16, c + 32, c + 48
@@ -131,7 +136,7 @@ __global__ __launch_bounds__(64 * kAttWaves, 2) void attention_mma_kernel(
     for (int b = 0; b < NB; ++b)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float p = expf(s[b][r] - ref);
+        const float p = expf(s[b][r] - ref) * kAttUnit;
         s[b][r] = p;
         ps += p;
       }
@@ -284,7 +289,7 @@ extern "C" int miq_attention(const float* q, const float* kcache, const float* v
   MIQ_REQUIRE(T >= 0 && NH > 0 && NKV > 0 && NH % NKV == 0 && HD > 0 && HD <= 256 && HD % 4 == 0 && LMAX > 0,
               MIQ_ERR_INVALID, "attention: T=%d NH=%d NKV=%d HD=%d LMAX=%d", T, NH, NKV, HD, LMAX);
   if (T == 0) return MIQ_OK;
-  MIQ_REQUIRE((size_t)LMAX * 4 <= 64 * 1024, MIQ_ERR_UNSUPPORTED, "attention: LMAX=%d above 16384", LMAX);
+  MIQ_REQUIRE(LMAX <= kAttMaxKeys, MIQ_ERR_UNSUPPORTED, "attention: LMAX=%d above %d", LMAX, kAttMaxKeys);
   MIQ_REQUIRE(q && kcache && vcache && state && out, MIQ_ERR_INVALID, "attention: null pointer");
   MIQ_REQUIRE(aligned(kcache, 16) && aligned(vcache, 16), MIQ_ERR_ALIGN, "attention: caches must be 16-byte aligned");
   const hipStream_t s = static_cast<hipStream_t>(stream);
