@@ -68,3 +68,15 @@ def test_gemv_workspace_query_is_host_only():
     assert core.gemv_workspace_bytes(0, 896, 4864, 128, 4, _lib.MIQ_F16) == 0
     with pytest.raises(NotImplementedError, match="group size"):
         core.gemv_workspace_bytes(1, 896, 4864, 16, 4, _lib.MIQ_F16)
+
+
+@pytest.mark.parametrize("dt,rows", [(_lib.MIQ_F16, 1), (_lib.MIQ_F32, 2)])
+def test_ggml_gemm_workspace_holds_sums_for_types_with_mins_only(dt, rows):
+    """The 8-byte sums of 32 staged values, which only Q4_K and Q5_K multiply (by their mins)."""
+    from webpytorch_amd import core
+    M, K, N = 1024, 4096, 14336  # a grid that does not split K
+    need = {t: core.ggml_gemm_workspace_bytes(M, K, N, dt, t)
+            for t in ("Q4_K", "Q5_K", "Q6_K", "Q8_0", "Q4_0", "Q5_0", "IQ4_NL")}
+    staged = rows * M * K * 2 + 4 * M + (4 << 20)
+    for t, n in need.items():
+        assert n == staged + (rows * M * K // 32 * 8 if t in ("Q4_K", "Q5_K") else 0), t

@@ -41,13 +41,13 @@
 //
 // fp32 activations enter as two fp16 rows each, hi = fp16(x 2^s) and lo = fp16(x 2^s - hi),
 // with 2^s per row putting the row's largest |x| near 2^15 (s = 0 for rows holding NaN or Inf);
-// the staging pass writes them and their sub-block sums as rows 2m and 2m + 1, and the GEMM's
+// the staging pass writes them as rows 2m and 2m + 1, and the GEMM's
 // epilogue adds the pair and scales back. fp16 activations are staged as they are.
 //
 // Staged rows: xs[r][k] fp16, each 8-wide k block in the order (0, 2, 1, 3, 4, 6, 5, 7) that
 // the code unpack produces (byte j of a code word holds value j, and one v_and_or_b32 takes
-// bytes 0 and 2, then 1 and 3); rs[r][k / 32] the sub-block sums of the staged fp16 values
-// (fp32, held as three bf16 and a zero whose sum is the fp32 value exactly).
+// bytes 0 and 2, then 1 and 3); rs[r][k / 32], for types with mins, the sub-block sums of the
+// staged fp16 values (fp32, held as three bf16 and a zero whose sum is the fp32 value exactly).
 //
 // Tiles: a workgroup of 4 waves computes 64 rows x 64 CG columns; wave w takes the CG groups of
 // 16 columns from 16 CG w and all 64 rows (four 16-row MFMA tiles per group). K is walked 256
@@ -110,18 +110,19 @@ __device__ __forceinline__ uint2 split_bf16(float v) {
 }
 
 // One workgroup per row m of x: rows R m .. R m + R - 1 of xs (R = 2 for fp32 x: hi, lo; 1 for
-// fp16) with their sub-block sums, and for fp32 the row's largest |x| (NaN if it holds one) in
-// rmax[m]. The four threads of a sub-block are consecutive (quad), so its sum is a quad sum.
+// fp16), for fp32 the row's largest |x| (NaN if it holds one) in rmax[m], and for types with mins
+// (SUMS) the rows' sub-block sums. The four threads of a sub-block are consecutive (quad), so its
+// sum is a quad sum.
 // Dynamic LDS K * 4 bytes for fp32 (the row is read once, its maximum sets the scale).
 //
 // NIB: the layout of the nibble types, whose code byte j of a 32-value block holds values j (low)
 // and 16 + j (high): chunk kb of a block holds values 4 kb .. + 3 and 16 + 4 kb .. + 3, so that a
 // lane's B operand is both nibbles of one dword.
-template <typename XT, bool NIB>
+template <typename XT, bool NIB, bool SUMS>
 __global__ __launch_bounds__(256) void stage_kernel(const XT* __restrict__ x, __half* __restrict__ xs,
                                                     uint2* __restrict__ rs, float* __restrict__ rmax, int K) {
   constexpr bool F32 = std::is_same<XT, float>::value;
-  const int m = blockIdx.x, nch = K / 8, K32 = K / 32;
+  const int m = blockIdx.x, nch = K / 8;
   float sc = 1.f;
   extern __shared__ __align__(16) float frow[];
   if constexpr (F32) {
@@ -177,12 +178,14 @@ __global__ __launch_bounds__(256) void stage_kernel(const XT* __restrict__ x, __
     }
     constexpr int R = F32 ? 2 : 1;
     *reinterpret_cast<uint4*>(xs + ((size_t)R * m) * K + 8 * i) = order8(hi);
-    const float shi = quad_sum(sum8(hi));
-    if ((i & 3) == 0) rs[((size_t)R * m) * K32 + i / 4] = split_bf16(shi);
-    if constexpr (F32) {
-      *reinterpret_cast<uint4*>(xs + ((size_t)R * m + 1) * K + 8 * i) = order8(lo);
-      const float slo = quad_sum(sum8(lo));
-      if ((i & 3) == 0) rs[((size_t)R * m + 1) * K32 + i / 4] = split_bf16(slo);
+    if constexpr (F32) *reinterpret_cast<uint4*>(xs + ((size_t)R * m + 1) * K + 8 * i) = order8(lo);
+    if constexpr (SUMS) {
+      const float shi = quad_sum(sum8(hi));
+      if ((i & 3) == 0) rs[((size_t)R * m) * (K / 32) + i / 4] = split_bf16(shi);
+      if constexpr (F32) {
+        const float slo = quad_sum(sum8(lo));
+        if ((i & 3) == 0) rs[((size_t)R * m + 1) * (K / 32) + i / 4] = split_bf16(slo);
+      }
     }
   }
 }
@@ -191,17 +194,17 @@ __global__ __launch_bounds__(256) void stage_kernel(const XT* __restrict__ x, __
 constexpr int kQ8_0 = 8, kQ4_K = 12, kQ5_K = 13, kQ6_K = 14;
 constexpr int kQ4_0 = 2, kQ5_0 = 6, kIQ4_NL = 20;  // the nibble types
 constexpr bool is_nib(int t) { return t == kQ4_0 || t == kQ5_0 || t == kIQ4_NL; }
+constexpr bool has_mins(int t) { return t == kQ4_K || t == kQ5_K; }
 
-// Per type: bytes per 256-value step, raw 32-bit registers per lane and step, whether the
-// sub-block mins (and so the row sums) enter.
+// Per type: bytes per 256-value step, raw 32-bit registers per lane and step.
 template <int T> struct KQ;
-template <> struct KQ<kQ4_K> { static constexpr int STEP = 144, RAW = 12; static constexpr bool MIN = true; };
-template <> struct KQ<kQ5_K> { static constexpr int STEP = 176, RAW = 14; static constexpr bool MIN = true; };
-template <> struct KQ<kQ6_K> { static constexpr int STEP = 210, RAW = 24; static constexpr bool MIN = false; };
-template <> struct KQ<kQ8_0> { static constexpr int STEP = 272, RAW = 32; static constexpr bool MIN = false; };
-template <> struct KQ<kQ4_0> { static constexpr int STEP = 144, RAW = 20; static constexpr bool MIN = false; };
-template <> struct KQ<kIQ4_NL> { static constexpr int STEP = 144, RAW = 20; static constexpr bool MIN = false; };
-template <> struct KQ<kQ5_0> { static constexpr int STEP = 176, RAW = 28; static constexpr bool MIN = false; };
+template <> struct KQ<kQ4_K> { static constexpr int STEP = 144, RAW = 12; };
+template <> struct KQ<kQ5_K> { static constexpr int STEP = 176, RAW = 14; };
+template <> struct KQ<kQ6_K> { static constexpr int STEP = 210, RAW = 24; };
+template <> struct KQ<kQ8_0> { static constexpr int STEP = 272, RAW = 32; };
+template <> struct KQ<kQ4_0> { static constexpr int STEP = 144, RAW = 20; };
+template <> struct KQ<kIQ4_NL> { static constexpr int STEP = 144, RAW = 20; };
+template <> struct KQ<kQ5_0> { static constexpr int STEP = 176, RAW = 28; };
 
 __device__ __forceinline__ uint32_t ld32(const uint8_t* p) { return *reinterpret_cast<const uint32_t*>(p); }
 __device__ __forceinline__ uint32_t ld16(const uint8_t* p) { return *reinterpret_cast<const unsigned short*>(p); }
@@ -361,7 +364,7 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(const __half* __restrict__
                                                    int Mx, int K, int N, int mtiles, int tiles, int ksteps,
                                                    float* __restrict__ part) {
   constexpr int RAW = KQ<T>::RAW, STEP = KQ<T>::STEP;
-  constexpr bool MIN = KQ<T>::MIN;
+  constexpr bool MIN = has_mins(T);
   __shared__ __align__(16) __half at[2][kBM * 256];  // activation tiles, 16-byte chunks swizzled by row
   // sub-block sums: 64 bytes a row, its 16-byte chunks (two sub-blocks each) swizzled by row / 4, so
   // that 16 rows of one chunk fall in different banks
@@ -676,15 +679,15 @@ static Plan plan(int M, int K, int N, int x_dtype) {
 struct Ws {
   size_t xs, rs, rmax, part, bytes;
 };
-// workspace layout after the shared counter region: staged rows, sub-block sums, row maxima,
-// K-slice partial sums
-static Ws layout(int M, int K, int N, int x_dtype) {
+// workspace layout after the shared counter region: staged rows, sub-block sums (types with mins),
+// row maxima, K-slice partial sums
+static Ws layout(int M, int K, int N, int x_dtype, int ggml_type) {
   const size_t R = x_dtype == MIQ_F32 ? 2 : 1, Mx = R * (size_t)M;
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
   Ws w;
   w.xs = kCounterBytes;
   w.rs = w.xs + up(Mx * K * 2);
-  w.rmax = w.rs + up(Mx * (K / 32) * 8);
+  w.rmax = w.rs + (has_mins(ggml_type) ? up(Mx * (K / 32) * 8) : 0);
   w.part = w.rmax + up((size_t)M * 4);
   const Plan p = plan(M, K, N, x_dtype);
   w.bytes = w.part + (p.ksplit > 1 ? up((size_t)p.ksplit * Mx * N * 4) : 0);
@@ -733,21 +736,21 @@ static int workspace_call(const char* who, bool ok, int M, int K, int N, int x_d
   MIQ_REQUIRE(ok, MIQ_ERR_UNSUPPORTED, "%s: ggml type %d has no GEMM", who, ggml_type);
   MIQ_REQUIRE(M >= 0 && K > 0 && N > 0 && K % 256 == 0, MIQ_ERR_INVALID, "%s: M=%d K=%d N=%d", who, M, K, N);
   MIQ_REQUIRE(x_dtype == MIQ_F16 || x_dtype == MIQ_F32, MIQ_ERR_UNSUPPORTED, "%s: x dtype", who);
-  *bytes = M == 0 ? 0 : layout(M, K, N, x_dtype).bytes;
+  *bytes = M == 0 ? 0 : layout(M, K, N, x_dtype, ggml_type).bytes;
   return MIQ_OK;
 }
 
-template <bool NIB>
+template <bool NIB, bool SUMS>
 static int stage(const void* x, int x_dtype, __half* xs, uint2* rs, float* rmax, int M, int K, hipStream_t st) {
   if (x_dtype == MIQ_F32) {
     if ((size_t)K * 4 > 64 * 1024) {
       const int rc = require_lds("ggml_gemm staging", (size_t)K * 4);
       if (rc) return rc;
     }
-    hipLaunchKernelGGL((stage_kernel<float, NIB>), dim3(M), dim3(256), (size_t)K * 4, st, static_cast<const float*>(x),
+    hipLaunchKernelGGL((stage_kernel<float, NIB, SUMS>), dim3(M), dim3(256), (size_t)K * 4, st, static_cast<const float*>(x),
                        xs, rs, rmax, K);
   } else {
-    hipLaunchKernelGGL((stage_kernel<__half, NIB>), dim3(M), dim3(256), 0, st, static_cast<const __half*>(x), xs, rs,
+    hipLaunchKernelGGL((stage_kernel<__half, NIB, SUMS>), dim3(M), dim3(256), 0, st, static_cast<const __half*>(x), xs, rs,
                        rmax, K);
   }
   return check_launch("ggml_gemm staging");
@@ -765,7 +768,7 @@ static int gemm_call(const char* who, bool ok, const void* x, int x_dtype, const
   MIQ_REQUIRE(x && w && out && workspace, MIQ_ERR_INVALID, "%s: null pointer", who);
   MIQ_REQUIRE(aligned(w, 16) && aligned(x, 16) && aligned(workspace, 256), MIQ_ERR_ALIGN,
               "%s: x and weight 16-byte, workspace 256-byte aligned", who);
-  const Ws L = layout(M, K, N, x_dtype);
+  const Ws L = layout(M, K, N, x_dtype, ggml_type);
   MIQ_REQUIRE(ws_bytes >= L.bytes, MIQ_ERR_INVALID, "%s: workspace %zu bytes, need %zu", who, ws_bytes, L.bytes);
   MIQ_REQUIRE(K <= 16384, MIQ_ERR_UNSUPPORTED, "%s: K=%d too large to stage", who, K);
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -774,8 +777,9 @@ static int gemm_call(const char* who, bool ok, const void* x, int x_dtype, const
   uint2* rs = reinterpret_cast<uint2*>(b + L.rs);
   float* rmax = reinterpret_cast<float*>(b + L.rmax);
   float* part = reinterpret_cast<float*>(b + L.part);
-  const int rc = is_nib(ggml_type) ? stage<true>(x, x_dtype, xs, rs, rmax, M, K, st)
-                                   : stage<false>(x, x_dtype, xs, rs, rmax, M, K, st);
+  const int rc = is_nib(ggml_type)    ? stage<true, false>(x, x_dtype, xs, rs, rmax, M, K, st)
+                 : has_mins(ggml_type) ? stage<false, true>(x, x_dtype, xs, rs, rmax, M, K, st)
+                                       : stage<false, false>(x, x_dtype, xs, rs, rmax, M, K, st);
   if (rc) return rc;
   switch (ggml_type) {
     case kQ4_K: return gemm_t<kQ4_K>(xs, rs, rmax, part, w, bias, out, out_dtype, M, x_dtype, K, N, st);
