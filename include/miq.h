@@ -131,6 +131,10 @@ int miq_gptq_gemv_fused(const float* x, int x_mode, const float* norm_w, float e
  * miq_gptq_gemv_workspace (zeroed counters first, not shared by concurrent calls). */
 int miq_gptq_gemm_workspace(int M, int K, int N, int gs, int bits, size_t* bytes);
 
+/* Bytes of workspace with which miq_gptq_gemm runs its few-row kernel on these rows in k order
+ * (perm NULL): 0 where it does not split K, SIZE_MAX where it does not cover the product. */
+int miq_gptq_gemm_few_rows_workspace(int M, int K, int N, int gs, int bits, size_t* bytes);
+
 /* Prefill / batched GEMM on the matrix cores: out[M][N] = x[M][K] (fp16, gathered through perm
  * if non-NULL) @ W + bias (nullable, fp32). W is dequantized exactly to the small integers
  * q - (z + zero_offset) in fp16 (zero_offset must be a small non-negative integer), fp16 x

@@ -87,3 +87,26 @@ def test_split_products_of_non_finite_and_huge_values(gpu, M, K, N):
     big[:128] *= 1e9
     got = product(sc, torch.from_numpy(x).cuda()).cpu().numpy()
     assert np.linalg.norm(got - x.astype(np.float64) @ big) < 3e-7 * np.linalg.norm(x.astype(np.float64) @ big)
+
+
+@pytest.mark.parametrize("M,K,N", [(6, 4096, 8136), (2, 4096, 11008)])
+def test_captured_products_are_the_eager_ones(gpu, M, K, N):
+    """A product that does not split K needs no workspace, so a capture on a stream without one
+    records the kernel that an eager call runs: every replay has the eager call's bits."""
+    import torch
+    from webpytorch_amd import core
+    L = synth.gptq_layer(M, K, N, 128, 4)
+    ql = core.QuantizedLinear.from_autogptq(L["qweight"], L["qzeros"], L["scales"], None, 128, 4)
+    x = torch.from_numpy(synth.activations(M, M, K, np.float16)).cuda()
+    eager = ql.forward(x)
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        out = ql.forward(x)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+        assert torch.equal(ql.forward(x), eager)

@@ -80,3 +80,15 @@ def test_ggml_gemm_workspace_holds_sums_for_types_with_mins_only(dt, rows):
     staged = rows * M * K * 2 + 4 * M + (4 << 20)
     for t, n in need.items():
         assert n == staged + (rows * M * K // 32 * 8 if t in ("Q4_K", "Q5_K") else 0), t
+
+
+def test_few_rows_workspace_says_what_the_kernel_covers():
+    """0 where K is not split, counters and fp32 slice sums where it is, None where another kernel
+    runs (more rows, other groups or code widths, more than 32 slices or 256 column tiles)."""
+    from webpytorch_amd import core
+    need = core.few_rows_workspace_bytes
+    assert need(6, 4096, 11008, 128, 4) == 0
+    assert need(6, 4096, 4096, 128, 4) == (4 << 20) + 8 * 64 * 4096  # slices x tiles x 16 x 64 floats
+    for M, K, N, gs, bits in ((17, 4096, 4096, 128, 4), (6, 4096, 4096, 64, 4), (6, 4096, 4096, 128, 8),
+                              (6, 16512, 512, 128, 4), (6, 8192, 16448, 128, 4)):
+        assert need(M, K, N, gs, bits) is None

@@ -108,6 +108,17 @@ def gemm_workspace_bytes(M, K, N, gs, bits):
     return b
 
 
+def few_rows_workspace_bytes(M, K, N, gs, bits):
+    """Bytes of workspace the few-row kernel behind `miq_gptq_gemm` needs for rows in k order, None
+    where it does not cover the product (cached per shape)."""
+    key = ("few", M, K, N, gs, bits)
+    if key not in _WS_BYTES:
+        n = ctypes.c_size_t(0)
+        _lib.call("miq_gptq_gemm_few_rows_workspace", M, K, N, gs, bits, ctypes.byref(n))
+        _WS_BYTES[key] = None if n.value == ctypes.c_size_t(-1).value else int(n.value)
+    return _WS_BYTES[key]
+
+
 def workspace(nbytes):
     """The split-K workspace of the current (device, stream), grown on demand and zeroed when
     allocated (the kernels leave its counter region zero). One workspace per stream: calls on
@@ -133,7 +144,7 @@ def workspace_holds(nbytes):
     """Whether the current stream's workspace already has nbytes."""
     dev = torch.cuda.current_device()
     t = _WORKSPACE.get((dev, torch.cuda.current_stream(dev).cuda_stream))
-    return t is not None and t.numel() >= nbytes
+    return nbytes == 0 or t is not None and t.numel() >= nbytes
 
 
 def aligned16(t):
@@ -215,21 +226,27 @@ def _gptq_path(M, xdt):
 # ---- GPTQ ----------------------------------------------------------------------------
 def _few_rows_gemm_taken(xf, qweight, scales, K, N, gs, bits, zoff, perm, ws):
     """Whether 2 to GEMV_MAX_M fp16 rows run on the few-row matrix-core kernel behind
-    `miq_gptq_gemm` rather than the GEMV, whose vector work grows with the rows. The shapes are
-    those that kernel covers (int4, groups of 128, rows in k order; at most 7680 outputs where it
-    splits K, which it does not for 8129 outputs and more with K to 4096). Both cost the host 18 us
+    `miq_gptq_gemm` rather than the GEMV, whose vector work grows with the rows. The kernel has to
+    cover the product (int4, groups of 128, rows in k order). Both cost the host 18 us
     a call; the GEMV's kernel passes that from about 2^25 products on (us a call, few-row / GEMV:
     4096 -> 4096 18 / 26 at 8 rows, 18 / 18 at 6; 4096 -> 11008 18 / 20 at 6; 11008 -> 4096 18 / 23
-    at 2, 18 / 50 at 8). A workspace handed in, or held while a graph is captured, has to suffice."""
+    at 2, 18 / 50 at 8). K to 16384, N to 7680 and, where K to 4096 leaves it unsplit, N from 8129
+    are the ranges the route was checked over, not limits of the kernel, which covers products past
+    them and is ahead there too (GPU us at 2 rows: 8192 -> 8192 13 / 22, 18944 -> 3584 16 / 37).
+    A workspace handed in has to suffice for `miq_gptq_gemm` whichever kernel it runs; while a graph
+    is captured the stream's has to hold what this kernel needs, which is nothing where K is not
+    split."""
     M = int(xf.shape[0])
     if not (1 < M <= GEMV_MAX_M and M * K * N >= FEW_ROWS_MIN and bits == 4 and gs == 128 and perm is None
             and xf.dtype == torch.float16 and float(zoff).is_integer() and 0 <= zoff <= 8 and K % 128 == 0
             and K <= 16384 and N % 8 == 0 and (N <= 7680 or (N > 8128 and K <= 4096))
             and qweight.data_ptr() % 16 == 0 and scales.data_ptr() % 16 == 0):
         return False
-    need = gemm_workspace_bytes(M, K, N, gs, bits)
+    need = few_rows_workspace_bytes(M, K, N, gs, bits)
+    if need is None:
+        return False
     if ws is not None:
-        return ws.numel() >= need and ws.data_ptr() % 256 == 0
+        return ws.numel() >= gemm_workspace_bytes(M, K, N, gs, bits) and ws.data_ptr() % 256 == 0
     return not torch.cuda.is_current_stream_capturing() or workspace_holds(need)
 
 
@@ -263,7 +280,7 @@ def _gptq_matmul(xf, qweight, qzeros, scales, K, N, gs, bits, zoff=0.0, *, bias=
     xd = dtype_code(xf)
     if few or M > GEMV_MAX_M and xd == MIQ_F16 and float(zoff).is_integer() and 0 <= zoff <= 8:
         if ws is None:
-            ws = workspace(gemm_workspace_bytes(M, K, N, gs, bits))
+            ws = workspace((few_rows_workspace_bytes if few else gemm_workspace_bytes)(M, K, N, gs, bits))
         _lib.call("miq_gptq_gemm", ptr(xf), ptr(perm), ptr(qweight), ptr(qzeros), ptr(scales),
                   dtype_code(scales), ptr(bias), ptr(out), dtype_code(out), M, K, N, gs, bits,
                   float(zoff), ptr(ws), 0 if ws is None else ws.numel(), stream_handle())

@@ -786,6 +786,15 @@ extern "C" int miq_gptq_gemm_workspace(int M, int K, int N, int gs, int bits, si
   return MIQ_OK;
 }
 
+extern "C" int miq_gptq_gemm_few_rows_workspace(int M, int K, int N, int gs, int bits, size_t* bytes) {
+  MIQ_REQUIRE(bytes, MIQ_ERR_INVALID, "gptq_gemm_few_rows_workspace: null output");
+  *bytes = SIZE_MAX;
+  int rc = check_gptq_dims("gptq_gemm_few_rows_workspace", K, N, gs, bits);
+  if (rc) return rc;
+  *bytes = gemm_small_workspace(M, K, N, gs, bits, false);
+  return MIQ_OK;
+}
+
 extern "C" int miq_gptq_gemm(const void* x, const int32_t* perm, const int32_t* qweight, const int32_t* qzeros,
                              const void* scales, int scales_dtype, const float* bias, void* out, int out_dtype, int M,
                              int K, int N, int gs, int bits, float zero_offset, void* workspace,
