@@ -35,7 +35,8 @@ namespace miq {
 // block's issued before the position is known) at short ones. Against one wave per (head,
 // token) with a score row in LDS, from position 0: 14 heads of 64, T = 64 6.1 -> 4.7 us, T = 700 138 -> 22,
 // T = 2000 997 -> 92; 28 heads of 128, T = 700 499 -> 58, T = 2000 4264 -> 339 (88 TFLOP/s); one
-// row behind 700 positions 37 -> 13 and 71 -> 19.
+// row behind 700 positions 37 -> 13 and 71 -> 19; up to 16 rows of heads of 64 lose 0.3-0.7 us there
+// (3.2-3.9 -> 4.0-4.2): half of a 32-key block is empty, and skipping it cost longer prompts more.
 constexpr int kAttWaves = 4;  // eight were slower from T = 700 on (T = 2000: 92 -> 106 us) and no faster below
 constexpr int kAttMaxKeys = 16384;           // LMAX
 constexpr float kAttUnit = 1.f / kAttMaxKeys;  // a probability of 1

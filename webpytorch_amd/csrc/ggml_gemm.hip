@@ -21,7 +21,7 @@
 //     MFMA per 16 x 16 tile and super-block (its 32 k slots are 8 sub-blocks x the 3 bf16 of a sum;
 //     the mins, below 64, are exact); d and dmin apply once per super-block. Before, two fp32
 //     MFMAs took the mins (a third of the matrix-core time) and every scale was cut out of its
-//     packed bytes on its own: 4096 -> 14336, 512 fp16 rows, 142 -> 108 us. What is left is the
+//     packed bytes on its own: 4096 -> 14336, 512 fp16 rows, 142 -> 108 us a call. What is left is the
 //     unpack (about 450 vector instructions against 72 MFMAs per wave and step) and the wait at
 //     each step's barrier with two waves a SIMD; tiles of 256 columns measured 5 % slower, loads
 //     spread over the sub-blocks no faster.
@@ -40,7 +40,8 @@
 // (plus the code offset), no conversion instruction per code.
 //
 // fp32 activations enter as two fp16 rows each, hi = fp16(x 2^s) and lo = fp16(x 2^s - hi),
-// with 2^s per row putting the row's largest |x| near 2^15 (s = 0 for rows holding NaN or Inf);
+// with 2^s per row putting the row's largest |x| near 2^15 (s = 0 for rows holding NaN or Inf): about
+// 22 of a value's 24 bits, with a floor of 2^-40 of the row's largest;
 // the staging pass writes them as rows 2m and 2m + 1, and the GEMM's
 // epilogue adds the pair and scales back. fp16 activations are staged as they are.
 //
@@ -309,8 +310,8 @@ __device__ __forceinline__ half2v byte_h2(uint32_t w, int j) {
   return as_h2(v) - (half2v){(_Float16)1024, (_Float16)1024};
 }
 // Four bytes of codes c in the bits of MASK of each byte (a nibble at bit 0 or 4) times an integer
-// scale, as two fp16 pairs (bytes 0, 2 and 1, 3): (1024 + c 2^k) s 2^-k - 1024 s 2^-k, one
-// rounding of an exact integer below 2048. w8 = w >> 8; s = scale 2^-k, off = -1024 s.
+// scale, as an fp16 pair (bytes 0 and 2 of w; of w >> 8, bytes 1 and 3): (1024 + c 2^k) s - 1024 s,
+// one rounding of an exact integer below 2048. s = scale 2^-k, off = -1024 s.
 template <uint32_t MASK> __device__ __forceinline__ half2v code_fma(uint32_t w, half2v s, half2v off) {
   return __builtin_elementwise_fma(as_h2(and_or(w, MASK | (MASK << 16), 0x64006400u)), s, off);
 }
