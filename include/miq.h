@@ -66,7 +66,8 @@ int miq_gptq_repack_rows(const int32_t* qweight, const int32_t* perm, int32_t* o
  * workspace (the counter region) hold arrival counters, fixed-point split-K sums and their
  * escape masks, shared by every split-K entry point, that must be zero before the first call
  * on it; every call leaves them zero again. Partial sums, escape slots and staged activations
- * follow them. One workspace must not serve two calls that run concurrently.
+ * follow them. One workspace must not serve two calls that run concurrently; calls that several
+ * threads make on one stream do not (each call enqueues all its kernels before the next one's).
  * The one-row int4 kernel sums its K-slices in fixed point on a grid of 2^-24, so outputs much
  * below 1 keep fewer digits (about 2^-24 per slice, whatever the output's size); a partial that is
  * NaN, infinite or of magnitude >= 2^22 (beyond the words) reaches the final sum as an fp32 value,

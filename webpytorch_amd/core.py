@@ -122,9 +122,10 @@ def few_rows_workspace_bytes(M, K, N, gs, bits):
 def workspace(nbytes):
     """The split-K workspace of the current (device, stream), grown on demand and zeroed when
     allocated (the kernels leave its counter region zero). One workspace per stream: calls on
-    one stream are ordered, so they never share it concurrently, and calls on two streams get
-    two workspaces. A grown workspace keeps the old one alive (a captured graph may still point
-    at it); growth at least doubles, so a stream retires O(log size) buffers."""
+    one stream are ordered, from several threads too, so they never share it concurrently, and
+    calls on two streams get two workspaces. A grown workspace keeps the old one alive (a captured
+    graph may still point at it); growth at least doubles, so a stream retires O(log size)
+    buffers."""
     if nbytes == 0:
         return None
     dev = torch.cuda.current_device()

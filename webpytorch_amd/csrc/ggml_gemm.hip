@@ -778,6 +778,7 @@ static int gemm_call(const char* who, bool ok, const void* x, int x_dtype, const
   uint2* rs = reinterpret_cast<uint2*>(b + L.rs);
   float* rmax = reinterpret_cast<float*>(b + L.rmax);
   float* part = reinterpret_cast<float*>(b + L.part);
+  std::lock_guard<std::mutex> whole(stream_lock(st));
   const int rc = is_nib(ggml_type)    ? stage<true, false>(x, x_dtype, xs, rs, rmax, M, K, st)
                  : has_mins(ggml_type) ? stage<false, true>(x, x_dtype, xs, rs, rmax, M, K, st)
                                        : stage<false, false>(x, x_dtype, xs, rs, rmax, M, K, st);

@@ -752,6 +752,7 @@ extern "C" int miq_gptq_gemm_f32x(const float* x, const int32_t* perm, const int
   float* rmax = reinterpret_cast<float*>(ws + p.rmax_off);
   const size_t lds = (size_t)K * 4;
   if (lds > 64 * 1024 && (rc = require_lds("gptq_gemm_f32x staging", lds))) return rc;
+  std::lock_guard<std::mutex> whole(stream_lock(st));
 #define MIQ_F32_STAGE(B, P)                                                                                      \
   hipLaunchKernelGGL((stage_rows_f32_kernel<B, P>), dim3(M), dim3(256), lds, st, x, perm, rmax, xp, M, K, p.g.kc)
   if (bits == 4) {
@@ -814,6 +815,7 @@ extern "C" int miq_gptq_gemm(const void* x, const int32_t* perm, const int32_t* 
   MIQ_REQUIRE(!perm || K <= 32768, MIQ_ERR_UNSUPPORTED, "gptq_gemm: act-order with K=%d > 32768", K);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const __half* xin = static_cast<const __half*>(x);
+  std::lock_guard<std::mutex> whole(stream_lock(st));
   // a few rows: the matrix-core kernel that streams the weights like the GEMV
   const size_t need_small = gemm_small_workspace(M, K, N, gs, bits, perm != nullptr);
   if (need_small != SIZE_MAX &&

@@ -4,6 +4,8 @@
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
+#include <mutex>
+
 #include "../../include/miq.h"
 
 namespace miq {
@@ -19,6 +21,15 @@ int require_lds(const char* what, size_t bytes);
   do {                                            \
     if (!(cond)) return ::miq::fail(code, __VA_ARGS__); \
   } while (0)
+
+// A call of several kernels that pass scratch to one another through the caller's workspace
+// enqueues them while it holds its stream's lock: a stream has one workspace, and between two of the
+// kernels another thread's call on the stream could enqueue its own and overwrite the scratch. The
+// lock ends with the call and waits for no kernel. Streams share 64 locks.
+inline std::mutex& stream_lock(hipStream_t st) {
+  static std::mutex locks[64];
+  return locks[(reinterpret_cast<uintptr_t>(st) >> 6) % 64];
+}
 
 inline bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
